@@ -2,11 +2,11 @@
 // solver 'RD1') on MI355X.
 //
 // compute_update_rd (:612-745) scatters four corner residuals of every quad
-// cell into its nodes.  Here each workgroup computes the corner values of the
-// cells around a tile of nodes into LDS and every node gathers its own, adding
-// them in the order the reference's cell loop (x outer, y inner) adds them, so
-// the sums round identically without atomics.  The two boundary passes apply
-// the reference's copies (:722-737) in their order.
+// cell into its nodes.  Here a wave marches up a strip of node columns, forms
+// each node's quantities once, each cell's corner residuals once, and every
+// node adds its own four in the order the reference's cell loop (x outer, y
+// inner) adds them, so the sums round identically without atomics.  The
+// reference's boundary copies (:722-737) are stores of the node they copy.
 // FP64 with contraction off and the reference's expression order throughout:
 // the results equal the oracle's bit for bit.
 #include <hip/hip_runtime.h>
@@ -19,10 +19,14 @@
 
 #include "../../include/fvwb.h"
 #include "fvwb_checkpoint.h"
+#include "fvwb_device.h"
 
 #pragma clang fp contract(off)
 
 namespace rd {
+
+using fvwb::lane_from_left;
+using fvwb::lane_from_right;
 
 struct Geo {
   int nx, ny, bc;
@@ -48,66 +52,8 @@ __device__ __forceinline__ void load4(const double* a, int nx, int i, int j, dou
   const double4 q = *reinterpret_cast<const double4*>(a + 4 * ((long long)j * nx + i));
   v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
 }
-
-// Corner residuals of cell (i, j) (nodes i..i+1, j..j+1): out[k*4 + v] for
-// corners k = 11, 12, 21, 22 (benchmark_rd.f90:653-697).
-__device__ __forceinline__ void cell_phi(const Geo& g, const double* __restrict__ u,
-                                         const double* __restrict__ diff, double dt, int i, int j,
-                                         double out[16]) {
-  double uu[4][4], ww[4][4], ff[4][4], gg[4][4], ss[4][4], sp[4];
-  load4(u, g.nx, i, j, uu[0]);
-  load4(u, g.nx, i + 1, j, uu[1]);
-  load4(u, g.nx, i, j + 1, uu[2]);
-  load4(u, g.nx, i + 1, j + 1, uu[3]);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    // compute_flux (:549-571): ff along x, gg along y
-    double w[4];
-    primitive(g.gamma, uu[k], w);
-    gg[k][0] = w[0] * w[2];
-    gg[k][1] = w[0] * w[1] * w[2];
-    gg[k][2] = w[2] * uu[k][2] + w[3];
-    gg[k][3] = w[2] * uu[k][3] + w[2] * w[3];
-    ff[k][0] = w[0] * w[1];
-    ff[k][1] = w[1] * uu[k][1] + w[3];
-    ff[k][2] = w[0] * w[1] * w[2];
-    ff[k][3] = w[1] * uu[k][3] + w[1] * w[3];
-    primitive(g.gamma, uu[k], ww[k]);
-    // get_source (:747-767), grad_p = (1, 1): it receives the primitive
-    // vector (:681-684) and converts it once more (:756), so its velocities
-    // are ww[1]/ww[0] and ww[2]/ww[0]
-    double w2[4];
-    primitive(g.gamma, ww[k], w2);
-    ss[k][0] = 0.0;
-    ss[k][1] = -w2[0] * 1.0;
-    ss[k][2] = -w2[0] * 1.0;
-    ss[k][3] = -w2[0] * (w2[1] * 1.0 + w2[2] * 1.0);
-    // the reference hands compute_speed the primitive vector (:692-695)
-    sp[k] = speed(g.gamma, ww[k]);
-  }
-  double alpha = sp[0];
-#pragma unroll
-  for (int k = 1; k < 4; ++k)
-    if (sp[k] > alpha) alpha = sp[k];
-  double dd[4][4];
-  load4(diff, g.nx, i, j, dd[0]);
-  load4(diff, g.nx, i + 1, j, dd[1]);
-  load4(diff, g.nx, i, j + 1, dd[2]);
-  load4(diff, g.nx, i + 1, j + 1, dd[3]);
-  const double dx = g.dx, dy = g.dy;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    // :673-678, corners 11, 12, 21, 22 = uu[0..3]
-    const double totalphi = -0.5 * (ff[0][v] + ff[2][v]) + 0.5 * (ff[1][v] + ff[3][v]) -
-                            0.5 * (gg[3][v] + gg[2][v]) + 0.5 * (gg[0][v] + gg[1][v]) -
-                            0.25 * (ss[0][v] + ss[2][v] + ss[1][v] + ss[3][v]) * dx * dy;
-    const double ubar = 0.25 * (uu[0][v] + uu[3][v] + uu[2][v] + uu[1][v]);
-    // :688-697
-    out[0 * 4 + v] = dy * dx * dd[0][v] * 0.25 + dt * (totalphi * 0.25 + alpha * (uu[0][v] - ubar) * dy);
-    out[1 * 4 + v] = dy * dx * dd[1][v] * 0.25 + dt * (totalphi * 0.25 + alpha * (uu[1][v] - ubar) * dy);
-    out[2 * 4 + v] = dy * dx * dd[2][v] * 0.25 + dt * (totalphi * 0.25 + alpha * (uu[2][v] - ubar) * dx);
-    out[3 * 4 + v] = dy * dx * dd[3][v] * 0.25 + dt * (totalphi * 0.25 + alpha * (uu[3][v] - ubar) * dx);
-  }
+__device__ __forceinline__ void store4(double* a, int nx, int i, int j, const double v[4]) {
+  *reinterpret_cast<double4*>(a + 4 * ((long long)j * nx + i)) = double4{v[0], v[1], v[2], v[3]};
 }
 
 // The resident time loop's clock, on the device so that steps follow each
@@ -119,81 +65,247 @@ struct Clock {
   int active, err;
 };
 
-// One workgroup per tile of TX x TY nodes: the corner residuals of the
-// (TX+1) x (TY+1) cells that touch the tile (its cells and a one-cell halo,
-// which the neighbouring tiles compute as well) go to LDS, then every node
-// gathers its up to four corner values from there in the order the
-// reference's x-outer, y-inner cell loop adds them (cells (a-1,b-1), (a-1,b),
-// (a,b-1), (a,b)), so the sums round as the reference's do and no corner value
-// travels through HBM.
-// 31 x 7 nodes make the 32 x 8 = 256 cells one per thread (one fill round).
-constexpr int TX = 31, TY = 7, CX = TX + 1, CY = TY + 1, NC = CX * CY;
-static_assert(NC == 256, "one cell per thread of the workgroup");
+// The node that the boundary copies make node `t` of 0..n-1 equal to, along x
+// (:722-729: the lower end first) and along y (:730-737: the upper end first).
+__host__ __device__ __forceinline__ int source_x(int bc, int n, int t) {
+  if (bc == FVWB_RD_BC_PERIODIC) return t == 0 ? n - 1 : t;
+  if (t == n - 1 && n > 2) return n - 2;
+  return t == 0 || n == 2 ? 1 : t;
+}
+__host__ __device__ __forceinline__ int source_y(int bc, int n, int t) {
+  if (bc == FVWB_RD_BC_PERIODIC) return t == n - 1 ? 0 : t;
+  if (t == 0 && n > 2) return 1;
+  return t == n - 1 || n == 2 ? n - 2 : t;
+}
 
-// dt is the argument, or the clock's when ck is given (the resident loop).
-__global__ __launch_bounds__(256) void rd_update_kernel(Geo g, const double* __restrict__ u,
-                                                        const double* __restrict__ diff, double dt,
-                                                        const Clock* __restrict__ ck, double* __restrict__ dudt) {
-  if (ck) {
+// What a cell needs of one of its nodes.
+struct Node {
+  double u[4], f[4], g[4];   // state, flux along x and along y
+  double s3, sp;             // energy source (the momentum ones are -u[0]), speed
+  double d[4];               // correction
+};
+
+__device__ __forceinline__ void node_values(double gamma, Node& n) {
+  // compute_flux (:549-571): f along x, g along y
+  double w[4], w2[4];
+  primitive(gamma, n.u, w);
+  n.g[0] = w[0] * w[2];
+  n.g[1] = w[0] * w[1] * w[2];
+  n.g[2] = w[2] * n.u[2] + w[3];
+  n.g[3] = w[2] * n.u[3] + w[2] * w[3];
+  n.f[0] = w[0] * w[1];
+  n.f[1] = w[1] * n.u[1] + w[3];
+  n.f[2] = w[0] * w[1] * w[2];
+  n.f[3] = w[1] * n.u[3] + w[1] * w[3];
+  // get_source (:747-767), grad_p = (1, 1): it receives the primitive vector
+  // (:681-684) and converts it once more (:756), so its velocities are
+  // w[1]/w[0] and w[2]/w[0]; compute_speed gets the primitive vector as well
+  // (:692-695)
+  primitive(gamma, w, w2);
+  n.s3 = -w2[0] * (w2[1] * 1.0 + w2[2] * 1.0);
+  const double cs = sqrt(gamma * fmax(w2[3], 1e-10) / fmax(w2[0], 1e-10));
+  n.sp = sqrt(w2[1] * w2[1] + w2[2] * w2[2]) + cs;
+}
+
+// UPDATE: dudt of (u, diff), the drop-in.  FIRST and SECOND are the two passes
+// of an 'RD1' step (evolve, :351-356) with their element-wise ends: FIRST has
+// diff = 0 and leaves up = u - dudt/(dx dy); SECOND has diff = up - u, leaves
+// the new u = up - dudt/(dx dy) and reduces its maximum speed.
+enum { UPDATE = 0, FIRST = 1, SECOND = 2 };
+
+constexpr int OWN = 62;                         // node columns a wave owns
+constexpr int SLOTS = 64, SLOT_STRIDE = 16;     // 16 x 8 B = one 128-byte line
+
+// A wave owns 62 node columns (lanes 1..62; lane l holds column x0 - 1 + l) and
+// `rows` node rows, and marches up them.  A lane forms the quantities of its
+// node of a row once, takes the node's on its right from the next lane (DPP),
+// and with the row below has everything of its cell (a, r-1); what a cell adds
+// to its right-hand nodes goes one lane on.  Each node's divisions and square
+// roots are so evaluated once (and once more in a strip's two halo rows and
+// columns), where a thread per cell evaluates them four times, and no value
+// goes through LDS.  At 2049^2 the two updates with their element-wise passes,
+// copies and speed pass took 570 us per step as separate kernels with a thread
+// per cell; see the launch rule in strip_rows() for what they take now.
+template <int MODE>
+__global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const double* __restrict__ u0,
+                                                       const double* __restrict__ u1, double* __restrict__ up,
+                                                       const double* __restrict__ diff, double dt, int rows,
+                                                       const Clock* __restrict__ ck, double* __restrict__ o0,
+                                                       double* __restrict__ o1,
+                                                       unsigned long long* __restrict__ smax) {
+  const double* u = u0;
+  double* out = o0;
+  if constexpr (MODE != UPDATE) {
     if (!ck->active) return;
     dt = ck->dt;
+    // the state alternates between two buffers, by the parity of the steps taken
+    const bool odd = ck->steps & 1;
+    u = odd ? u1 : u0;
+    out = MODE == FIRST ? up : (odd ? o0 : o1);
   }
-  __shared__ double lds[16 * NC];           // [corner*4 + v][cell], 32 KB
-  const int x0 = blockIdx.x * TX, y0 = blockIdx.y * TY;
-  const int c = threadIdx.x;                // cell (x0-1 + c%CX, y0-1 + c/CX)
-  const int ci = x0 - 1 + c % CX, cj = y0 - 1 + c / CX;
-  if (ci >= 0 && ci < g.nx - 1 && cj >= 0 && cj < g.ny - 1) {
-    double phi[16];
-    cell_phi(g, u, diff, dt, ci, cj, phi);
-#pragma unroll
-    for (int q = 0; q < 16; ++q) lds[q * NC + c] = phi[q];
-  }
-  __syncthreads();
-  const int tx = threadIdx.x % CX, ty = threadIdx.x / CX;   // node (x0+tx, y0+ty)
-  const int a = x0 + tx, b = y0 + ty;
-  if (tx >= TX || ty >= TY || a >= g.nx || b >= g.ny) return;
-  const int cx = g.nx - 1, cy = g.ny - 1;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  // local cell index of cell (a-1+di, b-1+dj) is (ty+dj)*CX + tx+di
-  auto add = [&](int di, int dj, int corner) {
-    const int c = (ty + dj) * CX + tx + di;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) s[v] = s[v] + lds[(corner * 4 + v) * NC + c];
+  const int lane = threadIdx.x & 63;
+  const int strips = (g.nx + OWN - 1) / OWN;
+  const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b0 = tile / strips * rows;
+  if (b0 >= g.ny) return;
+  const int b1 = min(b0 + rows, g.ny);
+  const int a = tile % strips * OWN - 1 + lane;          // this lane's node column
+  const int ac = min(max(a, 0), g.nx - 1);
+  const bool cell_x = a >= 0 && a < g.nx - 1;            // cell (a, .) exists
+  const bool own = lane >= 1 && lane <= OWN && a < g.nx;
+  // a strip that touches no end of the grid has no copies to make
+  const bool inner = b0 > 1 && b1 < g.ny - 1 && tile % strips > 0 && tile % strips * OWN + OWN < g.nx - 1;
+  const double dx = g.dx, dy = g.dy;
+
+  auto load = [&](int r, Node& n) {
+    const int rc = min(max(r, 0), g.ny - 1);
+    load4(u, g.nx, ac, rc, n.u);
+    if constexpr (MODE == UPDATE) load4(diff, g.nx, ac, rc, n.d);
+    if constexpr (MODE == SECOND) load4(up, g.nx, ac, rc, n.d);     // up itself until node() takes u off
   };
-  if (a >= 1 && b >= 1) add(0, 0, 3);
-  if (a >= 1 && b < cy) add(0, 1, 1);
-  if (a < cx && b >= 1) add(1, 0, 2);
-  if (a < cx && b < cy) add(1, 1, 0);
-  *reinterpret_cast<double4*>(dudt + 4 * ((long long)b * g.nx + a)) = double4{s[0], s[1], s[2], s[3]};
-}
+  auto node = [&](Node& n) {
+    node_values(g.gamma, n);
+  };
+  auto right4 = [&](const double v[4], double r[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = lane_from_right(v[k]);
+  };
+  // u - dudt/area of one node (or dudt itself) to node (ta, tb); base is the
+  // value that dudt is taken off
+  double speed_max = 0.0;
+  auto put = [&](int ta, int tb, const double s[4], const double base[4]) {
+    if constexpr (MODE == UPDATE) {
+      store4(out, g.nx, ta, tb, s);
+    } else {
+      double x[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[v] = base[v] - s[v] / area;
+      store4(out, g.nx, ta, tb, x);
+      if constexpr (MODE == SECOND) speed_max = fmax(speed_max, speed(g.gamma, x));
+    }
+  };
 
-__device__ __forceinline__ void copy_node(double* d, int nx, int ti, int tj, int si, int sj) {
-  double* t = d + 4 * ((long long)tj * nx + ti);
-  const double* s = d + 4 * ((long long)sj * nx + si);
-  t[0] = s[0]; t[1] = s[1]; t[2] = s[2]; t[3] = s[3];
-}
+  Node P, next;            // the row below, and the row in flight
+  double pr_u[4], pr_d[4], pr_s3, pr_sp;   // the row below: its right neighbour
+  double gsum[4];          // g of the row below plus its right neighbour's
+  double c2[4] = {0.0, 0.0, 0.0, 0.0}, c3[4] = {0.0, 0.0, 0.0, 0.0};   // corners of cell (a, r-2) at row r-1
+  double base[4];          // what dudt of row r-1 is taken off
+  load(b0 - 1, P);
+  load(b0, next);
+  auto settle = [&](Node& n, double b[4]) {
+    if constexpr (MODE == SECOND) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        b[v] = n.d[v];
+        n.d[v] = n.d[v] - n.u[v];
+      }
+    } else {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) b[v] = n.u[v];
+    }
+  };
+  settle(P, base);
+  node(P);
+  right4(P.u, pr_u);
+  if constexpr (MODE != FIRST) right4(P.d, pr_d);
+  pr_s3 = lane_from_right(P.s3);
+  pr_sp = lane_from_right(P.sp);
+#pragma unroll
+  for (int v = 0; v < 4; ++v) gsum[v] = P.g[v] + lane_from_right(P.g[v]);
 
-// :722-737, the copies along x (one thread per row j), then along y (one per column i)
-__global__ void rd_bc_x_kernel(Geo g, double* __restrict__ d) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= g.ny) return;
-  if (g.bc == FVWB_RD_BC_PERIODIC) {
-    copy_node(d, g.nx, 0, j, g.nx - 1, j);
-    copy_node(d, g.nx, g.nx - 1, j, 0, j);
-  } else {
-    copy_node(d, g.nx, 0, j, 1, j);
-    copy_node(d, g.nx, g.nx - 1, j, g.nx - 2, j);
+  // r: the row that closes cell row r-1 and completes node row r-1
+  for (int r = b0; r <= b1; ++r) {
+    Node N = next;
+    load(r + 1, next);
+    double nbase[4];
+    settle(N, nbase);
+    node(N);
+    double nr_u[4], nr_d[4], gs[4];
+    right4(N.u, nr_u);
+    if constexpr (MODE != FIRST) right4(N.d, nr_d);
+    const double nr_s3 = lane_from_right(N.s3), nr_sp = lane_from_right(N.sp);
+    const bool cell = cell_x && r >= 1 && r < g.ny;      // cell (a, r-1) exists
+    double alpha = P.sp;
+    if (pr_sp > alpha) alpha = pr_sp;
+    if (N.sp > alpha) alpha = N.sp;
+    if (nr_sp > alpha) alpha = nr_sp;
+    double q[4], k0[4], k2[4], k3[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      // :673-678, corners 11, 12, 21, 22 = P, its right neighbour, N, its right neighbour
+      gs[v] = N.g[v] + lane_from_right(N.g[v]);
+      const double fa = P.f[v] + N.f[v];
+      const double fb = lane_from_right(fa);
+      const double src = v == 0 ? 0.0
+                         : v == 3 ? P.s3 + N.s3 + pr_s3 + nr_s3
+                                  : -P.u[0] + -N.u[0] + -pr_u[0] + -nr_u[0];
+      const double totalphi = -0.5 * fa + 0.5 * fb - 0.5 * gs[v] + 0.5 * gsum[v] - 0.25 * src * dx * dy;
+      const double ubar = 0.25 * (P.u[v] + nr_u[v] + N.u[v] + pr_u[v]);
+      // :688-697
+      double k1;
+      if constexpr (MODE == FIRST) {
+        // diff = 0: its term is +0, which changes no sum that starts from +0
+        k0[v] = dt * (totalphi * 0.25 + alpha * (P.u[v] - ubar) * dy);
+        k1 = dt * (totalphi * 0.25 + alpha * (pr_u[v] - ubar) * dy);
+        k2[v] = dt * (totalphi * 0.25 + alpha * (N.u[v] - ubar) * dx);
+        k3[v] = dt * (totalphi * 0.25 + alpha * (nr_u[v] - ubar) * dx);
+      } else {
+        k0[v] = dy * dx * P.d[v] * 0.25 + dt * (totalphi * 0.25 + alpha * (P.u[v] - ubar) * dy);
+        k1 = dy * dx * pr_d[v] * 0.25 + dt * (totalphi * 0.25 + alpha * (pr_u[v] - ubar) * dy);
+        k2[v] = dy * dx * N.d[v] * 0.25 + dt * (totalphi * 0.25 + alpha * (N.u[v] - ubar) * dx);
+        k3[v] = dy * dx * nr_d[v] * 0.25 + dt * (totalphi * 0.25 + alpha * (nr_u[v] - ubar) * dx);
+      }
+      if (!cell) k0[v] = k1 = k2[v] = k3[v] = 0.0;
+      // what cell column a adds to node (a+1, r-1): cells (a, r-2) and (a, r-1)
+      q[v] = 0.0 + c3[v] + k1;
+    }
+    // node (a, r-1): cells (a-1, r-2), (a-1, r-1), (a, r-2), (a, r-1) in that
+    // order; a cell that does not exist counts as +0, which changes nothing
+    double s[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      s[v] = lane_from_left(q[v]) + c2[v] + k0[v];
+      c2[v] = k2[v];
+      c3[v] = k3[v];
+    }
+    const int b = r - 1;
+    if (b >= b0 && own) {
+      if (inner) {
+        put(a, b, s, base);
+      } else {
+        // every node whose value the copies take from this one: itself, and
+        // nodes of the four edges
+        const int xs[3] = {a, 0, g.nx - 1}, ys[3] = {b, 0, g.ny - 1};
+        for (int p = 0; p < 3; ++p) {
+          if (source_x(g.bc, g.nx, xs[p]) != a || (p > 0 && xs[p] == a) || (p == 2 && g.nx == 1)) continue;
+          for (int w = 0; w < 3; ++w) {
+            if (source_y(g.bc, g.ny, ys[w]) != b || (w > 0 && ys[w] == b)) continue;
+            if (MODE == UPDATE || (p == 0 && w == 0)) {
+              put(xs[p], ys[w], s, base);
+            } else {
+              double tb[4];
+              load4(MODE == FIRST ? u : up, g.nx, xs[p], ys[w], tb);
+              put(xs[p], ys[w], s, tb);
+            }
+          }
+        }
+      }
+    }
+    P = N;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      pr_u[v] = nr_u[v];
+      if constexpr (MODE != FIRST) pr_d[v] = nr_d[v];
+      gsum[v] = gs[v];
+      base[v] = nbase[v];
+    }
+    pr_s3 = nr_s3;
+    pr_sp = nr_sp;
   }
-}
-__global__ void rd_bc_y_kernel(Geo g, double* __restrict__ d) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= g.nx) return;
-  if (g.bc == FVWB_RD_BC_PERIODIC) {
-    copy_node(d, g.nx, i, g.ny - 1, i, 0);
-    copy_node(d, g.nx, i, 0, i, g.ny - 1);
-  } else {
-    copy_node(d, g.nx, i, g.ny - 1, i, g.ny - 2);
-    copy_node(d, g.nx, i, 0, i, 1);
+  if constexpr (MODE == SECOND) {
+    for (int off = 32; off > 0; off >>= 1) speed_max = fmax(speed_max, __shfl_xor(speed_max, off));
+    if (lane == 0)
+      atomicMax(smax + (blockIdx.x % SLOTS) * SLOT_STRIDE, (unsigned long long)__double_as_longlong(speed_max));
   }
 }
 
@@ -203,8 +315,6 @@ __global__ void rd_bc_y_kernel(Geo g, double* __restrict__ d) {
 // workgroup reduces its nodes and adds one atomicMax to one of SLOTS slots, a
 // cache line apart, so the atomics do not queue on one line; the host takes
 // the maximum of the slots.
-constexpr int SLOTS = 64, SLOT_STRIDE = 16;     // 16 x 8 B = one 128-byte line
-
 __global__ __launch_bounds__(256) void rd_speed_kernel(Geo g, const double* __restrict__ u,
                                                        unsigned long long* __restrict__ smax) {
   __shared__ double part[4];
@@ -225,18 +335,26 @@ __global__ __launch_bounds__(256) void rd_speed_kernel(Geo g, const double* __re
   }
 }
 
+// t = t + dt (:366), after a step that ran
+__device__ __forceinline__ void tick(Clock* ck) {
+  if (!ck->active) return;
+  ck->t = ck->t + ck->dt;
+  ck->dt_last = ck->dt;
+  ck->steps += 1;
+}
 // dt = min(cfl dx dy/cmax/3, t_end - t) (evolve, :348-349) from the speed
 // slots, which it clears for the next step; a maximum that is not finite and
-// positive stops the run with the error flag set.
-__global__ void rd_dt_kernel(Geo g, double cfl, double t_end, unsigned long long* __restrict__ smax,
-                             Clock* __restrict__ ck) {
+// positive stops the run with the error flag set.  One wave, a slot per lane;
+// `ticks` closes the step before this one first.
+__global__ __launch_bounds__(64) void rd_dt_kernel(Geo g, double cfl, double t_end, int ticks,
+                                                   unsigned long long* __restrict__ smax, Clock* __restrict__ ck) {
+  static_assert(SLOTS == 64, "a slot per lane");
+  const int k = threadIdx.x * SLOT_STRIDE;
+  double cmax = __longlong_as_double((long long)smax[k]);
+  smax[k] = 0;
+  for (int off = 32; off > 0; off >>= 1) cmax = fmax(cmax, __shfl_xor(cmax, off));
   if (threadIdx.x != 0) return;
-  unsigned long long m = 0;
-  for (int k = 0; k < SLOTS; ++k) {
-    m = max(m, smax[k * SLOT_STRIDE]);
-    smax[k * SLOT_STRIDE] = 0;
-  }
-  const double cmax = __longlong_as_double((long long)m);
+  if (ticks) tick(ck);
   if (ck->err || !(ck->t < t_end)) {
     ck->active = 0;
     return;
@@ -249,30 +367,8 @@ __global__ void rd_dt_kernel(Geo g, double cfl, double t_end, unsigned long long
   ck->dt = fmin(cfl * g.dy * g.dx / cmax / (2.0 * 1.0 + 1.0), t_end - ck->t);
   ck->active = 1;
 }
-// t = t + dt (:366), after the step
 __global__ void rd_tick_kernel(Clock* __restrict__ ck) {
-  if (threadIdx.x != 0 || !ck->active) return;
-  ck->t = ck->t + ck->dt;
-  ck->dt_last = ck->dt;
-  ck->steps += 1;
-}
-
-// up = u - dudt/(dx dy), diff = up - u (evolve, :351-354)
-__global__ void rd_pass1_kernel(long long n, double area, const double* __restrict__ u,
-                                const double* __restrict__ dudt, double* __restrict__ up,
-                                double* __restrict__ diff, const Clock* __restrict__ ck) {
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n || !ck->active) return;
-  const double x = u[k] - dudt[k] / area;
-  up[k] = x;
-  diff[k] = x - u[k];
-}
-// u = up - dudt/(dx dy) (:356)
-__global__ void rd_pass2_kernel(long long n, double area, double* __restrict__ u, const double* __restrict__ up,
-                                const double* __restrict__ dudt, const Clock* __restrict__ ck) {
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n || !ck->active) return;
-  u[k] = up[k] - dudt[k] / area;
+  if (threadIdx.x == 0) tick(ck);
 }
 
 }  // namespace rd
@@ -283,9 +379,9 @@ struct fvwb_rd {
   fvwb_rd_params p{};
   Geo g{};
   hipStream_t stream = nullptr;
-  double* d_u = nullptr;      // state, AoS(4,nx,ny)
+  double* buf[2] = {nullptr, nullptr};   // state, AoS(4,nx,ny): buf[par], the other one is the next step's
+  int par = 0;                           // parity of the clock's step count
   double* d_up = nullptr;
-  double* d_diff = nullptr;
   double* d_dudt = nullptr;
   unsigned long long* d_smax = nullptr;
   Clock* d_clk = nullptr;
@@ -311,7 +407,7 @@ extern "C" const char* fvwb_rd_last_error(fvwb_rd_handle h) { return h ? h->err.
 extern "C" int fvwb_rd_destroy(fvwb_rd_handle h) {
   if (!h) return FVWB_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  void* ps[] = {h->d_u, h->d_up, h->d_diff, h->d_dudt, h->d_smax, h->d_clk};
+  void* ps[] = {h->buf[0], h->buf[1], h->d_up, h->d_dudt, h->d_smax, h->d_clk};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -324,7 +420,7 @@ extern "C" int fvwb_rd_create(fvwb_rd_handle* out, const fvwb_rd_params* p) {
   *out = nullptr;
   if (p->nx < 2 || p->ny < 2) return failrd(nullptr, FVWB_ERR_ARG, "nx and ny must be >= 2");
   if ((long long)p->nx * p->ny > (1ll << 28)) return failrd(nullptr, FVWB_ERR_ARG, "more than 2^28 nodes");
-  if (p->ny > TY * 65535) return failrd(nullptr, FVWB_ERR_ARG, "ny must be <= 458745 (one grid row per 7 node rows)");
+  if (p->ny > 458745) return failrd(nullptr, FVWB_ERR_ARG, "ny must be <= 458745");
   if (p->bc != FVWB_RD_BC_PERIODIC && p->bc != FVWB_RD_BC_TRANSMISSIVE)
     return failrd(nullptr, FVWB_ERR_ARG, "bc must be 2 (periodic copies) or 3 (transmissive copies)");
   if (!(p->gamma > 1.0) || !(p->boxlen_x > 0.0) || !(p->boxlen_y > 0.0) || !(p->cfl > 0.0))
@@ -334,8 +430,8 @@ extern "C" int fvwb_rd_create(fvwb_rd_handle* out, const fvwb_rd_params* p) {
   h->p = *p;
   h->g = Geo{p->nx, p->ny, p->bc, p->gamma, p->boxlen_x / (double)(p->nx - 1), p->boxlen_y / (double)(p->ny - 1)};
   const size_t nb = sizeof(double) * 4 * (size_t)p->nx * (size_t)p->ny;
-  bool ok = hipStreamCreate(&h->stream) == hipSuccess && hipMalloc(&h->d_u, nb) == hipSuccess &&
-            hipMalloc(&h->d_up, nb) == hipSuccess && hipMalloc(&h->d_diff, nb) == hipSuccess &&
+  bool ok = hipStreamCreate(&h->stream) == hipSuccess && hipMalloc(&h->buf[0], nb) == hipSuccess &&
+            hipMalloc(&h->buf[1], nb) == hipSuccess && hipMalloc(&h->d_up, nb) == hipSuccess &&
             hipMalloc(&h->d_dudt, nb) == hipSuccess &&
             hipMalloc(&h->d_smax, sizeof(unsigned long long) * SLOTS * SLOT_STRIDE) == hipSuccess &&
             hipMalloc(&h->d_clk, sizeof(Clock)) == hipSuccess;
@@ -347,12 +443,27 @@ extern "C" int fvwb_rd_create(fvwb_rd_handle* out, const fvwb_rd_params* p) {
   return FVWB_OK;
 }
 
-// dudt of compute_update_rd for the device state u and correction diff.
-static int update(fvwb_rd* h, const double* u, const double* diff, double dt, const Clock* ck, double* dudt) {
-  const dim3 grid((unsigned)((h->p.nx + TX - 1) / TX), (unsigned)((h->p.ny + TY - 1) / TY));
-  hipLaunchKernelGGL(rd_update_kernel, grid, dim3(256), 0, h->stream, h->g, u, diff, dt, ck, dudt);
-  hipLaunchKernelGGL(rd_bc_x_kernel, dim3((unsigned)((h->p.ny + 255) / 256)), dim3(256), 0, h->stream, h->g, dudt);
-  hipLaunchKernelGGL(rd_bc_y_kernel, dim3((unsigned)((h->p.nx + 255) / 256)), dim3(256), 0, h->stream, h->g, dudt);
+// Rows of a strip: about 4096 strips (two rounds of the two waves per SIMD that
+// SECOND runs at), between 2 and 12 rows each.  A strip marches 2 rows more than
+// it owns, so short ones repeat work and long ones leave the chip idle on small
+// grids.  Measured us per step with 2 / 4 / 8 / 12 / 16 / 24 rows: 129^2 18.8 /
+// 24.6 / 37.3 / 49.9 / 62.7 / 87.3, 513^2 35.2 / 37.7 / 39.7 / 51.7 / 64.4 /
+// 89.1, 1025^2 80.4 / 73.1 / 77.2 / 75.7 / 93.5 / 90.1, 2049^2 275 / 231 / 209 /
+// 201 / 211 / 205.
+static int strip_rows(const Geo& g) {
+  const long long strips = (g.nx + OWN - 1) / OWN;
+  return (int)std::max(2LL, std::min(12LL, strips * g.ny / 4096));
+}
+
+// One sweep: dudt of (u0, diff) into o0, or a pass of an 'RD1' step between the
+// state's two buffers.
+template <int MODE>
+static int sweep(fvwb_rd* h, const double* u0, const double* u1, double* up, const double* diff, double dt,
+                 const Clock* ck, double* o0, double* o1) {
+  const int rows = strip_rows(h->g);
+  const long long tiles = (long long)((h->p.nx + OWN - 1) / OWN) * ((h->p.ny + rows - 1) / rows);
+  hipLaunchKernelGGL(rd_sweep_kernel<MODE>, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, h->stream, h->g,
+                     h->g.dx * h->g.dy, u0, u1, up, diff, dt, rows, ck, o0, o1, h->d_smax);
   HIPR(h, hipGetLastError());
   return FVWB_OK;
 }
@@ -383,8 +494,9 @@ extern "C" int fvwb_rd_compute_update(fvwb_rd_handle h, const double* u, const d
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
   // the update works in the step's scratch arrays; an uploaded state stays as it is
   HIPR(h, hipMemcpyAsync(h->d_up, u, nb, hipMemcpyHostToDevice, h->stream));
-  HIPR(h, hipMemcpyAsync(h->d_diff, diff, nb, hipMemcpyHostToDevice, h->stream));
-  int rc = update(h, h->d_up, h->d_diff, dt, nullptr, h->d_dudt);
+  double* d_diff = h->buf[h->par ^ 1];
+  HIPR(h, hipMemcpyAsync(d_diff, diff, nb, hipMemcpyHostToDevice, h->stream));
+  int rc = sweep<UPDATE>(h, h->d_up, nullptr, nullptr, d_diff, dt, nullptr, h->d_dudt, nullptr);
   if (rc) return rc;
   HIPR(h, hipMemcpyAsync(dudt, h->d_dudt, nb, hipMemcpyDeviceToHost, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
@@ -402,7 +514,8 @@ extern "C" int fvwb_rd_upload(fvwb_rd_handle h, const double* u) {
   if (!h || !u) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
   const Clock zero{};
-  HIPR(h, hipMemcpyAsync(h->d_u, u, nb, hipMemcpyHostToDevice, h->stream));
+  h->par = 0;
+  HIPR(h, hipMemcpyAsync(h->buf[0], u, nb, hipMemcpyHostToDevice, h->stream));
   HIPR(h, hipMemcpyAsync(h->d_clk, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
   h->loaded = true;
@@ -412,6 +525,7 @@ extern "C" int fvwb_rd_upload(fvwb_rd_handle h, const double* u) {
 static int read_clock(fvwb_rd* h, Clock* c) {
   HIPR(h, hipMemcpyAsync(c, h->d_clk, sizeof *c, hipMemcpyDeviceToHost, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
+  h->par = (int)(c->steps & 1);
   return FVWB_OK;
 }
 
@@ -426,28 +540,24 @@ extern "C" int fvwb_rd_advance(fvwb_rd_handle h, int32_t nsteps, double t_end) {
   if (!h) return failrd(h, FVWB_ERR_ARG, "NULL handle");
   if (!h->loaded) return failrd(h, FVWB_ERR_STATE, "advance before upload");
   if (nsteps < 0) return failrd(h, FVWB_ERR_ARG, "nsteps must be >= 0");
-  const long long n = 4ll * h->p.nx * h->p.ny;
-  const double area = h->g.dx * h->g.dy;
-  const dim3 eb(256), eg((unsigned)((n + 255) / 256));
-  HIPR(h, hipMemsetAsync(h->d_smax, 0, sizeof(unsigned long long) * SLOTS * SLOT_STRIDE, h->stream));
   Clock c{};
   int rc = read_clock(h, &c);
   if (rc) return rc;
+  // the state's maximum speed; every step leaves its new state's
+  HIPR(h, hipMemsetAsync(h->d_smax, 0, sizeof(unsigned long long) * SLOTS * SLOT_STRIDE, h->stream));
+  launch_speed(h, h->buf[h->par]);
+  double *b0 = h->buf[0], *b1 = h->buf[1];
   int32_t done = 0;
   while (done < nsteps && !c.err && c.t < t_end) {
     const int32_t k = std::min(kGroup, nsteps - done);
     for (int32_t s = 0; s < k; ++s) {
-      launch_speed(h, h->d_u);
-      hipLaunchKernelGGL(rd_dt_kernel, dim3(1), dim3(64), 0, h->stream, h->g, h->p.cfl, t_end, h->d_smax, h->d_clk);
-      HIPR(h, hipMemsetAsync(h->d_diff, 0, sizeof(double) * (size_t)n, h->stream));
-      if ((rc = update(h, h->d_u, h->d_diff, 0.0, h->d_clk, h->d_dudt))) return rc;
-      hipLaunchKernelGGL(rd_pass1_kernel, eg, eb, 0, h->stream, n, area, h->d_u, h->d_dudt, h->d_up, h->d_diff,
-                         h->d_clk);
-      if ((rc = update(h, h->d_u, h->d_diff, 0.0, h->d_clk, h->d_dudt))) return rc;
-      hipLaunchKernelGGL(rd_pass2_kernel, eg, eb, 0, h->stream, n, area, h->d_u, h->d_up, h->d_dudt, h->d_clk);
-      hipLaunchKernelGGL(rd_tick_kernel, dim3(1), dim3(64), 0, h->stream, h->d_clk);
-      HIPR(h, hipGetLastError());
+      hipLaunchKernelGGL(rd_dt_kernel, dim3(1), dim3(64), 0, h->stream, h->g, h->p.cfl, t_end, s > 0 ? 1 : 0,
+                         h->d_smax, h->d_clk);
+      if ((rc = sweep<FIRST>(h, b0, b1, h->d_up, nullptr, 0.0, h->d_clk, nullptr, nullptr))) return rc;
+      if ((rc = sweep<SECOND>(h, b0, b1, h->d_up, nullptr, 0.0, h->d_clk, b0, b1))) return rc;
     }
+    hipLaunchKernelGGL(rd_tick_kernel, dim3(1), dim3(64), 0, h->stream, h->d_clk);
+    HIPR(h, hipGetLastError());
     done += k;
     if ((rc = read_clock(h, &c))) return rc;
   }
@@ -459,7 +569,7 @@ extern "C" int fvwb_rd_download(fvwb_rd_handle h, double* u) {
   if (!h || !u) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   if (!h->loaded) return failrd(h, FVWB_ERR_STATE, "download before upload");
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
-  HIPR(h, hipMemcpyAsync(u, h->d_u, nb, hipMemcpyDeviceToHost, h->stream));
+  HIPR(h, hipMemcpyAsync(u, h->buf[h->par], nb, hipMemcpyDeviceToHost, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -468,7 +578,7 @@ extern "C" int fvwb_rd_download(fvwb_rd_handle h, double* u) {
 extern "C" int fvwb_rd_checkpoint_save(fvwb_rd_handle h, const char* path) {
   if (!h || !path) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   if (!h->loaded) return failrd(h, FVWB_ERR_STATE, "checkpoint before upload");
-  const fvwb_ckpt::Segment seg[2] = {{h->d_u, sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny},
+  const fvwb_ckpt::Segment seg[2] = {{h->buf[h->par], sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny},
                                      {h->d_clk, sizeof(Clock)}};
   std::string err;
   const int rc = fvwb_ckpt::save(path, fvwb_ckpt::RD, &h->p, sizeof h->p, 0, seg, 2, h->stream, err);
@@ -478,14 +588,23 @@ extern "C" int fvwb_rd_checkpoint_save(fvwb_rd_handle h, const char* path) {
 
 extern "C" int fvwb_rd_checkpoint_load(fvwb_rd_handle h, const char* path) {
   if (!h || !path) return failrd(h, FVWB_ERR_ARG, "NULL argument");
-  const fvwb_ckpt::Segment seg[2] = {{h->d_u, sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny},
+  const fvwb_ckpt::Segment seg[2] = {{h->buf[0], sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny},
                                      {h->d_clk, sizeof(Clock)}};
   std::string err;
   int32_t parity = 0;
   const int rc = fvwb_ckpt::load(path, fvwb_ckpt::RD, &h->p, sizeof h->p, &parity, seg, 2, h->stream, err);
   h->loaded = rc == FVWB_OK;
-  if (rc) h->err = err;
-  return rc;
+  h->par = 0;
+  if (rc) {
+    h->err = err;
+    return rc;
+  }
+  // the state lies in buf[0]; the clock's step count says which of the two it is
+  Clock c{};
+  const int rc2 = read_clock(h, &c);
+  if (rc2) return rc2;
+  if (h->par) std::swap(h->buf[0], h->buf[1]);
+  return FVWB_OK;
 }
 
 extern "C" int fvwb_rd_get_time(fvwb_rd_handle h, double* t, double* dt_last, int64_t* steps) {

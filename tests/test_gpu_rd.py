@@ -67,6 +67,31 @@ def test_run_matches_oracle(ninit, bc):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("bc", [fvwb.RD_BC_TRANSMISSIVE, fvwb.RD_BC_PERIODIC])
+@pytest.mark.parametrize("shape", [(2, 2), (3, 2), (2, 3), (62, 3), (63, 4), (64, 5), (125, 2), (187, 25), (5, 300)])
+def test_strip_edges_and_buffer_parity(shape, bc, tmp_path):
+    """Grids that end at, before and after a strip's 62 columns and its rows,
+    runs cut after an odd step, a drop-in call between them, and a checkpoint
+    of an odd step count loaded into a fresh handle."""
+    nx, ny = shape
+    say(f"case: rd strip edges {nx}x{ny} bc={bc}")
+    gp, op = params(nx, ny, bc, cfl=0.1)
+    u0 = random_state(nx, ny, nx * 7 + ny)
+    ref, t, n = po.rd_run(op, u0, np.inf, 5)
+    path = str(tmp_path / "rd.ckpt")
+    with fvwb.SolverRD(gp) as s, fvwb.SolverRD(gp) as r:
+        s.upload(u0)
+        s.advance(3)
+        np.testing.assert_array_equal(s.compute_update(u0, u0, 1e-3), po.rd_update(op, u0, u0, 1e-3))
+        s.checkpoint_save(path)
+        r.checkpoint_load(path)
+        for h in (s, r):
+            h.advance(1)
+            h.advance(1)
+            assert h.time()[0] == t and h.time()[2] == n == 5
+            np.testing.assert_array_equal(h.download(), ref)
+
+
 def test_t_end_clip_and_resume():
     """advance stops at t_end exactly, as evolve's dt = min(..., tend - t) does,
     and two advances equal one."""
