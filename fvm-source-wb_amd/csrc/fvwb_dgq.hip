@@ -9,33 +9,20 @@
 // only +, -, *, /, sqrt, min and max, written in the reference's order with
 // contraction off, so they round as the reference's do.
 //
-// One residual evaluation (compute_update, :1137-1479) is three launches:
-//   dgq_trace_kernel  one thread per cell: the traces at xi = -1, +1 and
-//                     eta = -1, +1 (:1253-1314) and their fluxes
-//                     (compute_flux_int :946-965), written face-major so that
-//                     the face pass reads them coalesced;
-//   dgq_face_kernel   one thread per face point: compute_num_flux (:991-1006)
-//                     between the traces of the two cells, with the
-//                     reference's get_boundary_conditions(., 2) indexing;
-//   dgq_cell_kernel   one thread per cell: node values, volume integrals,
-//                     edge integrals, source, assembly (:1448-1466),
-//                     special_boundary_conditions, and, for the resident time
-//                     loop, the Runge-Kutta stage combination of evolve in
-//                     the reference's expression order.
-// dgq_limit_kernel is compute_positivity (2d/limiters.f90:478-654) per cell;
-// the dgq_speed_*_kernels are compute_max_speed (:826-870) with its
-// bookkeeping and evolve's dt (:671), as exact block reductions.
+// A stage of evolve, with its residual (compute_update, :1137-1479), its
+// combination and its limiter (compute_positivity, 2d/limiters.f90:478-654), is
+// one launch of dgq_stage_kernel; the dgq_speed_*_kernels are compute_max_speed
+// (:826-870) with its bookkeeping and evolve's dt (:671), as exact block
+// reductions.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
-#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <string>
-#include <utility>
 
 #include "../../include/fvwb.h"
 
@@ -43,6 +30,9 @@
 
 namespace dgq {
 
+#ifndef DGQ_WAVES
+#define DGQ_WAVES 3
+#endif
 constexpr int MAXO = 3;
 
 // Basis and quadrature of one set-up (order O = mx = my).
@@ -68,21 +58,19 @@ struct Clock {
   int active, err;
 };
 
-// One Runge-Kutta stage of evolve: out = ((a0 X0 + a1 X1) + ...) + (cdt dt) L,
-// the reference's left-to-right order; nterms = 0 writes L itself.  With part
-// set, the stage also stores part = (b0 Y0 + b1 Y1) + ... (npart terms: the
-// leading terms of a later stage that takes the same L) and lval = L, so that
-// the later stage finishes from them instead of evaluating L again.
+// One Runge-Kutta stage of evolve: out = (a X + am in) + (cdt dt) L, in that
+// order, X or (own = 0) the stage's input absent from the sum; combine = 0
+// writes L itself.  limit applies compute_positivity to the result.  With w5
+// set, the stage also leaves w5 = ((b0 X + b1 Y) + bm in) + b4 out + (c5 dt) L,
+// the last combination of 'RK4' and 'SS4' that takes the same L (the reference
+// evaluates it twice, :700 and :723).  tick closes the step.
 struct Epi {
-  const double* X[4];
-  double a[4];
-  double cdt;
-  int nterms;
-  const double* Y[3];
-  double b[3];
-  int npart;
-  double* part;
-  double* lval;
+  const double* X;
+  double a, am, cdt;
+  int combine, own, limit, tick;
+  double* w5;
+  const double* Y;
+  double b0, b1, bm, b4, c5;
 };
 
 // ---- host: 2d/legendre.f90 as the reference evaluates it ------------------------
@@ -215,19 +203,22 @@ __device__ __forceinline__ void speed(double gamma, const double u[4], double& c
 
 // compute_num_flux (:991-1006); flag 1 along x, 2 along y.  A flux_type of no
 // branch (the shipped 'llf') and an HLLC state of no branch leave out at zero,
-// the value the reference's F and G start from (:1317-1318).
-__device__ void num_flux(const Geo& g, const double ul[4], const double ur[4], const double fl[4],
+// the value the reference's F and G start from (:1317-1318).  HLLC is an
+// instantiation of its own: its star states hold the stage kernel's registers
+// (O = 2: 142 against 114, a wave per SIMD less).
+template <bool HLLC>
+__device__ __forceinline__ void num_flux(const Geo& g, const double ul[4], const double ur[4], const double fl[4],
                          const double fr[4], int flag, double out[4]) {
   out[0] = out[1] = out[2] = out[3] = 0.0;
   const double gamma = g.gamma;
-  if (g.flux == FVWB_DGQ_FLUX_LLF1) {            // compute_llflux (:968-988)
+  if (!HLLC && g.flux == FVWB_DGQ_FLUX_LLF1) {            // compute_llflux (:968-988)
     double csl, vxl, vyl, spl, csr, vxr, vyr, spr;
     speed(gamma, ul, csl, vxl, vyl, spl);
     speed(gamma, ur, csr, vxr, vyr, spr);
     const double cmax = flag == 1 ? fmax_r(fabs(vxr + csr), fabs(vxl + csl)) : fmax_r(fabs(vyr + csr), fabs(vyl + csl));
 #pragma unroll
     for (int v = 0; v < 4; ++v) out[v] = 0.5 * (fr[v] + fl[v]) + 0.5 * cmax * (ul[v] - ur[v]);
-  } else if (g.flux == FVWB_DGQ_FLUX_HLL2) {     // compute_hllflux (:1008-1026)
+  } else if (!HLLC && g.flux == FVWB_DGQ_FLUX_HLL2) {     // compute_hllflux (:1008-1026)
     double csl, vxl, vyl, spl, csr, vxr, vyr, spr;
     speed(gamma, ul, csl, vxl, vyl, spl);
     speed(gamma, ur, csr, vxr, vyr, spr);
@@ -235,7 +226,7 @@ __device__ void num_flux(const Geo& g, const double ul[4], const double ur[4], c
     const double am = fmax_r(0.0, fmax_r(-(csl - sqrt(vxl * vxl + vyl * vyl)), -(csr - sqrt(vxr * vxr + vyr * vyr))));
 #pragma unroll
     for (int v = 0; v < 4; ++v) out[v] = (ap * fl[v] + am * fr[v] - ap * am * (ur[v] - ul[v])) / (ap + am);
-  } else if (g.flux == FVWB_DGQ_FLUX_HLLC) {     // compute_hllcflux (:1030-1134) as written
+  } else if (HLLC) {     // compute_hllcflux (:1030-1134) as written
     double wl[4], wr[4], csl, vxl, vyl, spl, csr, vxr, vyr, spr;
     prim(gamma, ul, wl);
     prim(gamma, ur, wr);
@@ -325,269 +316,121 @@ __device__ __forceinline__ long long at(int v, long long c, long long nc, int a,
   return (long long)v + 4 * (c + nc * ((long long)a + O * b));
 }
 
-// Trace buffer: states then fluxes, element ((side*O + q)*4 + v)*nc + c with
-// side 0 = left (xi = -1), 1 = right, 2 = bottom (eta = -1), 3 = top; the
-// flux of a left/right trace is the x flux, of a bottom/top trace the y flux.
+// Lane layout of the stage and limiter kernels: lane 4 col + v holds the modes
+// of variable v of the wave's cell col, which is the order of the arrays, so
+// every load and store of a wave is one run of 16 cells x 4 variables.  Where a
+// point needs all four variables (a node's fluxes, a pressure), the four lanes
+// of a cell pass their values through a few KB of LDS of their own wave and
+// take one point each.
+constexpr int TX = 16;                             // cells of a wave, and of a tile in x
+
+// orders a wave's own LDS writes before its other lanes' reads (and the reverse);
+// the LDS serves one wave's accesses in order, so only the compiler is held
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ void get4(const double* s, double u[4]) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) u[v] = s[v];
+}
+__device__ __forceinline__ void put4(double* s, const double u[4]) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v) s[v] = u[v];
+}
+
+// Products with the basis values.  Three exact properties of make_tab's values
+// spare multiplications and registers without changing a result: the constant
+// mode's value is 1; the points and weights are mirrored, so that mode n at the
+// mirrored point is (-1)^n times its value here; and gll_quadrature's outer
+// points are the cell's edges.  A product at a mirrored point is written as the
+// sign of the other one, and the compiler forms it once.
+// x legendre(x_quad(a), n)
 template <int O>
-__global__ __launch_bounds__(256) void dgq_trace_kernel(Geo g, Tab T, const double* __restrict__ du,
-                                                        double* __restrict__ tr, const Clock* __restrict__ ck) {
-  if (ck && !ck->active) return;
-  const long long nc = (long long)g.nx * g.ny;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nc) return;
-  double m[4][O][O];
+__device__ __forceinline__ double times_l(const Tab& T, double x, int a, int n) {
+  if (n == 0) return x;
+  const bool mirror = a > (O - 1) / 2;
+  const double r = x * T.L[mirror ? O - 1 - a : a][n];
+  return mirror && n % 2 == 1 ? -r : r;
+}
+// the same for a point known only at run time
+__device__ __forceinline__ double times_row(const Tab& T, double x, int a, int n) { return n == 0 ? x : x * T.L[a][n]; }
+// x legendre(-1, n) or x legendre(+1, n)
+__device__ __forceinline__ double times_edge(const Tab& T, double x, bool plus, int n) {
+  if (n == 0) return x;
+  const double r = x * T.lp[n];
+  return !plus && n % 2 == 1 ? -r : r;
+}
+// x legendre(x_gll(c), n)
+__device__ __forceinline__ double times_g(const Tab& T, double x, int c, int n) {
+  if (n == 0) return x;
+  return c == 1 ? x * T.Gl[1][n] : times_edge(T, x, c == 2, n);
+}
+// x legendre_prime(x_quad(a), n) w_quad(a), n >= 1
+template <int O>
+__device__ __forceinline__ double times_pw(const Tab& T, double x, int a, int n) {
+  const bool mirror = a > (O - 1) / 2;
+  const int k = mirror ? O - 1 - a : a;
+  const double r = x * T.P[n == 1 ? 0 : k][n];
+  return (mirror && n % 2 == 0 ? -r : r) * T.wq[k];
+}
+template <int O>
+__device__ __forceinline__ double weight(const Tab& T, int a) {
+  return T.wq[a > (O - 1) / 2 ? O - 1 - a : a];
+}
+
+// sum over the modes, i outer and j inner, of second(first(m[i][j])), in the
+// reference's order of the factors
+template <int O, class First, class Second>
+__device__ __forceinline__ double expand(const double m[O][O], First first, Second second) {
+  double s = 0.0;
 #pragma unroll
   for (int i = 0; i < O; ++i)
 #pragma unroll
-    for (int j = 0; j < O; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) m[v][i][j] = du[at<O>(v, c, nc, i, j)];
-  double* fl = tr + 16LL * O * nc;
-#pragma unroll
-  for (int side = 0; side < 4; ++side) {
-#pragma unroll
-    for (int q = 0; q < O; ++q) {
-      double s[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int i = 0; i < O; ++i)
-#pragma unroll
-        for (int j = 0; j < O; ++j)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            // :1259-1266 (x sides) and :1288-1297 (y sides)
-            const double b1 = side == 0 ? T.lm[i] : side == 1 ? T.lp[i] : side == 2 ? T.lm[j] : T.lp[j];
-            const double b2 = side < 2 ? T.L[q][j] : T.L[q][i];
-            s[v] = s[v] + m[v][i][j] * b1 * b2;
-          }
-      double f[4];
-      flux_int(g.gamma, s, side < 2 ? 0 : 1, f);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        tr[((long long)(side * O + q) * 4 + v) * nc + c] = s[v];
-        fl[((long long)(side * O + q) * 4 + v) * nc + c] = f[v];
-      }
-    }
-  }
+    for (int j = 0; j < O; ++j) s = s + second(first(m[i][j], i, j), i, j);
+  return s;
 }
-
-// Face fluxes: x faces F(v, q, f, j) at ((f + (nx+1) j) O + q) 4 + v, f = 0..nx;
-// y faces G(v, q, i, f) at ((i + nx f) O + q) 4 + v, f = 0..ny.
+// the trace at point q of a cell's x edge, of a cell's y edge, and the value at node (a, b)
 template <int O>
-__global__ __launch_bounds__(256) void dgq_face_kernel(Geo g, const double* __restrict__ tr,
-                                                       double* __restrict__ F, double* __restrict__ G,
-                                                       const Clock* __restrict__ ck) {
-  if (ck && !ck->active) return;
-  const long long nc = (long long)g.nx * g.ny;
-  const long long nfx = (long long)(g.nx + 1) * g.ny * O, nfy = (long long)g.nx * (g.ny + 1) * O;
-  long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nfx + nfy) return;
-  const double* fl = tr + 16LL * O * nc;
-  const bool xdir = k < nfx;
-  if (!xdir) k -= nfx;
-  const int q = (int)(k % O);
-  const long long r = k / O;
-  long long cl, cr;
-  int sl, sr;
-  if (xdir) {
-    const int f = (int)(r % (g.nx + 1)), j = (int)(r / (g.nx + 1));
-    const int il = bc_index(f, g.ny, g.bc) - 1, ir = bc_index(f + 1, g.ny, g.bc) - 1;
-    cl = il + (long long)g.nx * j;       // right trace of the left cell
-    cr = ir + (long long)g.nx * j;       // left trace of the right cell
-    sl = 1;
-    sr = 0;
-  } else {
-    const int i = (int)(r % g.nx), f = (int)(r / g.nx);
-    const int jl = bc_index(f, g.ny, g.bc) - 1, jr = bc_index(f + 1, g.ny, g.bc) - 1;
-    cl = i + (long long)g.nx * jl;       // top trace of the cell below
-    cr = i + (long long)g.nx * jr;       // bottom trace of the cell above
-    sl = 3;
-    sr = 2;
-  }
-  double ul[4], ur[4], ful[4], fur[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    ul[v] = tr[((long long)(sl * O + q) * 4 + v) * nc + cl];
-    ur[v] = tr[((long long)(sr * O + q) * 4 + v) * nc + cr];
-    ful[v] = fl[((long long)(sl * O + q) * 4 + v) * nc + cl];
-    fur[v] = fl[((long long)(sr * O + q) * 4 + v) * nc + cr];
-  }
-  double out[4];
-  num_flux(g, ul, ur, ful, fur, xdir ? 1 : 2, out);
-  double* dst = (xdir ? F : G) + 4 * k;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) dst[v] = out[v];
+__device__ __forceinline__ double trace_x(const Tab& T, const double m[O][O], bool plus, int q) {
+  return expand<O>(m, [&](double x, int i, int) { return times_edge(T, x, plus, i); },
+                   [&](double x, int, int j) { return times_l<O>(T, x, q, j); });
 }
-
-// The residual of one cell, one variable at a time (the node values and
-// fluxes are recomputed per variable so the accumulators of one variable fit
-// in registers), then the stage combination.  Accumulation orders are the
-// reference's: over the nodes a outer, b inner for the volume and source
-// integrals, over the face points for the edges.  The residual of the
-// block's cells waits in LDS until all four variables are done: for a node
-// (i, j) the block's cells and variables are one contiguous run of the
-// output (element v + 4 (c + nc (i + O j))), which the block then combines
-// and stores in full cache lines.
-constexpr int CELL_THREADS = 128;
-
 template <int O>
-__global__ __launch_bounds__(CELL_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void dgq_cell_kernel(
-    Geo g, Tab T, const double* __restrict__ in, const double* __restrict__ x, const double* __restrict__ y,
-    const double* __restrict__ F, const double* __restrict__ G, Epi e, double* out, const Clock* __restrict__ ck) {
-  if (ck && !ck->active) return;
-  __shared__ double sres[O * O * CELL_THREADS * 4];
-  const long long nc = (long long)g.nx * g.ny;
-  const long long c0 = (long long)blockIdx.x * CELL_THREADS;
-  const int tid = threadIdx.x;
-  const long long c = c0 + tid;
-  const double dt = ck ? ck->dt : 0.0;
-  if (c < nc) {
-    const int ic = (int)(c % g.nx), jc = (int)(c / g.nx);
-    double m[4][O][O];
-#pragma unroll
-    for (int i = 0; i < O; ++i)
-#pragma unroll
-      for (int j = 0; j < O; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) m[v][i][j] = in[at<O>(v, c, nc, i, j)];
-    const double odx = g.odx;
-    // two variables per pass: the nodal state and its fluxes, which every
-    // variable needs, are formed once for the pair; each accumulator still
-    // takes its terms in the reference's order
-#pragma unroll 1
-    for (int vp = 0; vp < 4; vp += 2) {
-      double fv1[2][O][O], fv2[2][O][O], sv[2][O][O];
-#pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int i = 0; i < O; ++i)
-#pragma unroll
-          for (int j = 0; j < O; ++j) fv1[r][i][j] = fv2[r][i][j] = sv[r][i][j] = 0.0;
-      // the node loops stay rolled: unrolled, the kernel held every table entry
-      // and node value at once (496 VGPRs, one wave per SIMD); the order of the
-      // sums is the same either way
-#pragma unroll 1
-      for (int a = 0; a < O; ++a)
-#pragma unroll 1
-        for (int b = 0; b < O; ++b) {
-          // get_nodes_from_modes (:544-592): modes a' outer, b' inner
-          double u[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-          for (int ma = 0; ma < O; ++ma)
-#pragma unroll
-            for (int mb = 0; mb < O; ++mb)
-#pragma unroll
-              for (int w = 0; w < 4; ++w) u[w] = u[w] + m[w][ma][mb] * T.L[a][ma] * T.L[b][mb];
-          double f1[4], f2[4];
-          flux_full(g.gamma, u, f1, f2);
-          double s[2] = {0.0, 0.0};
-          bool has_s = false;
-          if (g.source == 2) {                     // get_source (:1558-1576)
-            double w[4], g0, g1;
-            prim(g.gamma, u, w);
-            grad_phi(g.gpc, x[c + nc * (a + O * b)], y[c + nc * (a + O * b)], g0, g1);
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-              const int v = vp + r;
-              s[r] = v == 0 ? 0. : v == 1 ? w[0] * g0 : v == 2 ? w[0] * g1 : w[0] * (w[1] * g0 + w[2] * g1);
-            }
-            has_s = true;
-          } else if (g.source == 3) {              // get_adv_source (:1579-1596)
-#pragma unroll
-            for (int r = 0; r < 2; ++r) s[r] = vp + r == 0 ? -1.0 * u[0] : 0.0;
-            has_s = true;
-          }
-#pragma unroll
-          for (int r = 0; r < 2; ++r)
-#pragma unroll
-            for (int i = 0; i < O; ++i)
-#pragma unroll
-              for (int j = 0; j < O; ++j) {
-                fv1[r][i][j] = fv1[r][i][j] + f1[vp + r] * T.P[a][i] * T.wq[a] * T.L[b][j] * T.wq[b];
-                fv2[r][i][j] = fv2[r][i][j] + f2[vp + r] * T.P[b][j] * T.wq[b] * T.L[a][i] * T.wq[a];
-                if (has_s) sv[r][i][j] = sv[r][i][j] + s[r] * T.L[a][i] * T.wq[a] * T.L[b][j] * T.wq[b];
-              }
-        }
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        const int v = vp + r;
-        // face values of this variable: F at the cell's left (ic) and right
-        // (ic+1) x faces, G at its bottom (jc) and top (jc+1) y faces
-        double fr[O], fle[O], gt[O], gb[O];
-#pragma unroll
-        for (int q = 0; q < O; ++q) {
-          fle[q] = F[4 * (((long long)ic + (long long)(g.nx + 1) * jc) * O + q) + v];
-          fr[q] = F[4 * (((long long)ic + 1 + (long long)(g.nx + 1) * jc) * O + q) + v];
-          gb[q] = G[4 * (((long long)ic + (long long)g.nx * jc) * O + q) + v];
-          gt[q] = G[4 * (((long long)ic + (long long)g.nx * (jc + 1)) * O + q) + v];
-        }
-#pragma unroll
-        for (int i = 0; i < O; ++i)
-#pragma unroll
-          for (int j = 0; j < O; ++j) {
-            double e1 = 0.0, e2 = 0.0, e3 = 0.0, e4 = 0.0;
-#pragma unroll
-            for (int q = 0; q < O; ++q) {          // :1377-1386
-              e1 = e1 + fr[q] * T.lp[i] * T.L[q][j] * T.wq[q];
-              e2 = e2 + fle[q] * T.lm[i] * T.L[q][j] * T.wq[q];
-            }
-#pragma unroll
-            for (int q = 0; q < O; ++q) {          // :1391-1408
-              e3 = e3 + gt[q] * T.lp[j] * T.L[q][i] * T.wq[q];
-              e4 = e4 + gb[q] * T.lm[j] * T.L[q][i] * T.wq[q];
-            }
-            // :1455-1462 (oneoverdx for the y terms too)
-            double d = (odx * fv1[r][i][j] + odx * fv2[r][i][j] - odx * (e1 - e2) - odx * (e3 - e4)) / 2. +
-                       sv[r][i][j] / 4.;
-            if (g.ninit == 12) {                   // special_boundary_conditions (:1481-1514)
-              const double xd = x[c + nc * (i + O * j)] - g.boxlen_x / 2.;
-              const double yd = y[c + nc * (i + O * j)] - g.boxlen_y / 2.;
-              if (sqrt(xd * xd + yd * yd) > 2.0) d = 0.0;
-            }
-            sres[((i + O * j) * CELL_THREADS + tid) * 4 + v] = d;
-          }
-      }
-    }
-  }
-  __syncthreads();
-  // node (i, j): elements [4 (c0 + nc (i + O j)), + 4 ncells) of every array
-  const int ncell = (int)(nc - c0 < CELL_THREADS ? nc - c0 : CELL_THREADS);
-#pragma unroll 1
-  for (int ij = 0; ij < O * O; ++ij) {
-    const long long base = 4 * (c0 + nc * ij);
-    for (int q = tid; q < 4 * ncell; q += CELL_THREADS) {
-      const long long idx = base + q;
-      const double d = sres[ij * CELL_THREADS * 4 + q];
-      if (e.nterms == 0) {
-        out[idx] = d;
-      } else {
-        double sacc = e.a[0] * e.X[0][idx];
-        for (int k = 1; k < e.nterms; ++k) sacc = sacc + e.a[k] * e.X[k][idx];
-        out[idx] = sacc + e.cdt * dt * d;
-        if (e.part) {
-          double pacc = e.b[0] * e.Y[0][idx];
-          for (int k = 1; k < e.npart; ++k) pacc = pacc + e.b[k] * e.Y[k][idx];
-          e.part[idx] = pacc;
-          e.lval[idx] = d;
-        }
-      }
-    }
-  }
+__device__ __forceinline__ double trace_y(const Tab& T, const double m[O][O], bool plus, int q) {
+  return expand<O>(m, [&](double x, int, int j) { return times_edge(T, x, plus, j); },
+                   [&](double x, int i, int) { return times_l<O>(T, x, q, i); });
+}
+template <int O>
+__device__ __forceinline__ double node_value(const Tab& T, const double m[O][O], int a, int b) {
+  return expand<O>(m, [&](double x, int i, int) { return times_row(T, x, a, i); },
+                   [&](double x, int, int j) { return times_l<O>(T, x, b, j); });
 }
 
-// The rest of a stage whose leading terms and L a previous stage stored (Epi
-// part / lval): out = (part + a X) + (cdt dt) L, the same operations in the
-// same order as the stage evaluated in one piece.  out may alias part.
-__global__ __launch_bounds__(256) void dgq_finish_kernel(long long n, const double* part, double a,
-                                                         const double* __restrict__ X, double cdt,
-                                                         const double* __restrict__ lval, double* out,
-                                                         const Clock* __restrict__ ck) {
-  if (!ck->active) return;
-  const double dt = ck->dt;
-  for (long long idx = (long long)blockIdx.x * 256 + threadIdx.x; idx < n; idx += (long long)gridDim.x * 256) {
-    double sacc = part[idx];
-    sacc = sacc + a * X[idx];
-    out[idx] = sacc + cdt * dt * lval[idx];
-  }
+// Mode (i, j) of a lane: a plane that is the same for the whole wave plus the
+// lane's byte offset 8 (v + 4 c), which stays below 2^30 (2^24 cells).  One
+// 32-bit register then addresses every plane of every array; as 64-bit indexes
+// per plane the compiler kept 18 registers of addresses through the kernel.
+template <int O>
+__device__ __forceinline__ double& mode(double* u, unsigned lane_at, long long nc, int i, int j) {
+  return *(double*)((char*)(u + 4 * nc * (i + O * j)) + lane_at);
+}
+template <int O>
+__device__ __forceinline__ double mode(const double* u, unsigned lane_at, long long nc, int i, int j) {
+  return *(const double*)((const char*)(u + 4 * nc * (i + O * j)) + lane_at);
+}
+template <int O>
+__device__ __forceinline__ void load_modes(const double* __restrict__ u, unsigned lane_at, long long nc, double m[O][O]) {
+#pragma unroll
+  for (int j = 0; j < O; ++j)
+#pragma unroll
+    for (int i = 0; i < O; ++i) m[i][j] = mode<O>(u, lane_at, nc, i, j);
+}
+// element k of a per-cell array
+__device__ __forceinline__ double cell_value(const double* plane, unsigned k) {
+  return *(const double*)((const char*)plane + 8u * k);
 }
 
 // solve_for_t (2d/limiters.f90:312-362): the root in [0,1] of the quadratic
@@ -612,80 +455,436 @@ __device__ double solve_for_t(double gamma, double eps, const double u[4], const
   return t;
 }
 
-// compute_set (2d/limiters.f90:438-475), point k of 2 O gll: the first O gll
-// points at (x_gll(c), y_gl(q)), k = q gll + c, the others at (x_gl(q), y_gll(c))
+// compute_set's points (2d/limiters.f90:438-475): O x O at (x_gll(c), y_gl(q)),
+// k = q O + c, then O x O at (x_gl(q), y_gll(c)); gll_quadrature gives O points
 template <int O>
-__device__ __forceinline__ void set_point(const Tab& T, const double m[4][O][O], int k, double p[4]) {
-  const int half = O * T.gll;
-  const bool second = k >= half;
-  const int kk = second ? k - half : k;
-  const int q = kk / T.gll, cg = kk % T.gll;
-  p[0] = p[1] = p[2] = p[3] = 0.0;
-#pragma unroll
-  for (int i = 0; i < O; ++i)
-#pragma unroll
-    for (int j = 0; j < O; ++j) {
-      const double bi = second ? T.L[q][i] : T.Gl[cg][i];
-      const double bj = second ? T.Gl[cg][j] : T.L[q][j];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) p[v] = p[v] + m[v][i][j] * bi * bj;
-    }
+__device__ __forceinline__ double set_value(const Tab& T, const double m[O][O], int k) {
+  const int q = k % (O * O) / O, c = k % O;
+  return k < O * O ? expand<O>(m, [&](double x, int i, int) { return times_g(T, x, c, i); },
+                               [&](double x, int, int j) { return times_l<O>(T, x, q, j); })
+                   : expand<O>(m, [&](double x, int i, int) { return times_l<O>(T, x, q, i); },
+                               [&](double x, int, int j) { return times_g(T, x, c, j); });
 }
 
-// compute_positivity (2d/limiters.f90:478-654) on one cell, in place: theta
-// over the set's densities scales the non-mean density modes, then the
-// smallest solve_for_t over the set points whose pressure (density floored at
-// the default-real 10e-10) is not above eps scales every non-mean mode.
+// compute_positivity (2d/limiters.f90:478-654) on the wave's 16 cells, m in the
+// lane layout above: theta over the set's densities scales the non-mean density
+// modes, then the smallest solve_for_t over the set points whose pressure
+// (density floored at the default-real 10e-10) is not above eps scales every
+// non-mean mode.  Both minima are exact, so the points may go in any order.
+// The second minimum is formed beside the first, as if theta were 1; only a
+// wave that has a theta below 1 goes over the set again with its scaled density.
+struct LimitLds {
+  double pts[4][TX][4];                            // four set points x cells x variables
+  double avg[TX][4];
+};
+
 template <int O>
-__global__ __launch_bounds__(256) void dgq_limit_kernel(Geo g, Tab T, double* __restrict__ u,
-                                                        const Clock* __restrict__ ck) {
-  if (ck && !ck->active) return;
-  const long long nc = (long long)g.nx * g.ny;
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= nc) return;
-  double m[4][O][O];
-#pragma unroll
-  for (int i = 0; i < O; ++i)
-#pragma unroll
-    for (int j = 0; j < O; ++j)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) m[v][i][j] = u[at<O>(v, c, nc, i, j)];
-  const int np = 2 * O * T.gll;
+__device__ void limit_cells(const Geo& g, const Tab& T, LimitLds& s, double m[O][O]) {
+  constexpr int NP = 2 * O * O;
+  const int lane = threadIdx.x & 63, col = lane >> 2, v = lane & 3;
   const double eps = g.eps, gamma = g.gamma;
-  {
+  double theta = 1.0, tmin = 1.;
+  s.avg[col][v] = m[0][0];
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
     double pmin = 0.0;
-    for (int k = 0; k < np; ++k) {
-      double p[4];
-      set_point<O>(T, m, k, p);
-      pmin = k == 0 ? p[0] : fmin(pmin, p[0]);
+#pragma unroll
+    for (int k0 = 0; k0 < NP; k0 += 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (k0 + k < NP) {
+          const double p = set_value<O>(T, m, k0 + k);
+          pmin = k0 + k == 0 ? p : fmin(pmin, p);
+          s.pts[k][col][v] = p;
+        }
+      wave_lds_sync();
+      if (k0 + v < NP) {
+        double q[4];
+        get4(s.pts[v][col], q);
+        const double r = fmax(q[0], (double)10e-10f);
+        const double vx = q[1] / r, vy = q[2] / r;
+        const double pr = (gamma - 1.0) * (q[3] - 0.5 * r * (vx * vx + vy * vy));
+        double t = 1.;
+        if (!(pr > eps)) {
+          double avg[4];
+          get4(s.avg[col], avg);
+          t = solve_for_t(gamma, eps, q, avg);
+        }
+        if (tmin >= t) tmin = t;
+      }
+      wave_lds_sync();
+      __builtin_amdgcn_sched_barrier(0);           // a few values at a time
     }
-    const double theta = fmin(fabs((m[0][0][0] - eps) / (m[0][0][0] - pmin)), 1.0);
+    if (pass == 0 && v == 0) theta = fmin(fabs((m[0][0] - eps) / (m[0][0] - pmin)), 1.0);
+    if (pass == 1 || !__any(theta != 1.0)) break;
+    tmin = 1.;
 #pragma unroll
     for (int i = 0; i < O; ++i)
 #pragma unroll
       for (int j = 0; j < O; ++j)
-        if (i != 0 || j != 0) m[0][i][j] = theta * m[0][i][j];
+        if (i != 0 || j != 0) m[i][j] = theta * m[i][j];
   }
-  const double avg[4] = {m[0][0][0], m[1][0][0], m[2][0][0], m[3][0][0]};
-  double tmin = 1.;
-  for (int k = 0; k < np; ++k) {
-    double p[4];
-    set_point<O>(T, m, k, p);
-    const double r = fmax(p[0], (double)10e-10f);
-    const double vx = p[1] / r, vy = p[2] / r;
-    const double pr = (gamma - 1.0) * (p[3] - 0.5 * r * (vx * vx + vy * vy));
-    const double t = pr > eps ? 1. : solve_for_t(gamma, eps, p, avg);
+#pragma unroll
+  for (int x = 1; x < 4; x <<= 1) {
+    const double t = __shfl_xor(tmin, x);
     if (tmin >= t) tmin = t;
   }
 #pragma unroll
   for (int i = 0; i < O; ++i)
 #pragma unroll
     for (int j = 0; j < O; ++j)
+      if (i != 0 || j != 0) m[i][j] = tmin * m[i][j];
+}
+
+template <int O>
+__global__ __launch_bounds__(256) void dgq_limit_kernel(Geo g, Tab T, double* __restrict__ u) {
+  __shared__ LimitLds s[4];
+  const long long nc = (long long)g.nx * g.ny;
+  const int w = threadIdx.x >> 6, v = threadIdx.x & 3;
+  const long long c = (long long)blockIdx.x * (4 * TX) + (threadIdx.x >> 2);
+  double m[O][O];
+  const unsigned la = 8u * (unsigned)(v + 4 * (c < nc ? c : nc - 1));   // lanes past the end repeat the last cell
+  load_modes<O>(u, la, nc, m);
+  limit_cells<O>(g, T, s[w], m);
+  if (c >= nc) return;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const double val = (i != 0 || j != 0) ? tmin * m[v][i][j] : m[v][i][j];
-        u[at<O>(v, c, nc, i, j)] = val;
+  for (int j = 0; j < O; ++j)
+#pragma unroll
+    for (int i = 0; i < O; ++i) mode<O>(u, la, nc, i, j) = m[i][j];
+}
+
+// grad_phi at the nodes: it depends on the coordinates alone, so the resident
+// loop forms it once per upload
+__global__ __launch_bounds__(256) void dgq_grad_kernel(int gcase, long long n, const double* __restrict__ x,
+                                                       const double* __restrict__ y, double* __restrict__ gx,
+                                                       double* __restrict__ gy) {
+  const long long k = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (k < n) grad_phi(gcase, x[k], y[k], gx[k], gy[k]);
+}
+
+// One stage on a tile of TX x TY cells, a wave per row of 16 cells:
+//   1. every lane expands its variable's modes to the cell's four traces
+//      (:1253-1314); waves 0 to 2 also do the one trace that each neighbour of
+//      the tile owes it (get_boundary_conditions at the domain's edge);
+//   2. a thread per face point: the traces' fluxes (compute_flux_int :946-965)
+//      and compute_num_flux, written over the lower trace, which no other
+//      thread reads;
+//   3. O (or, for O = 2, all four) nodes at a time: node values, fluxes and
+//      source by one lane per node, then every lane adds them to its variable's
+//      volume and source integrals, a outer, b inner;
+//   4. edge integrals, assembly (:1448-1466), special_boundary_conditions, the
+//      Runge-Kutta combination, compute_positivity, and for the fourth 'RK4'
+//      stage w5.
+// Every sum takes its terms in the reference's order.
+//
+// Bound by FP64 issue: about 2,800 vector instructions per wave, 63 % of the
+// issue slots at 512^2 and O = 3, 2.2 TB/s.  One launch instead of the four
+// (traces, faces, cells, limiter) that moved 400 MB of traces and face fluxes
+// and the state three more times per stage: 125 against 390 us per stage at
+// 512^2, 8 against 32 at 16^2.  Tiles of 16 x 8 cells share more halo but hold
+// twice the waves at each barrier: 165 us.  Four waves per SIMD (128
+// registers) against three: 4 % faster.
+template <int O, int TY>
+struct StageLds {
+  static constexpr int NB = O == 2 ? 4 : O;        // nodes per pass
+  double yt[O][TY + 1][TX][4];                     // top traces of rows -1 .. TY-1, then the y face fluxes
+  double xr[O][TY][TX + 1][4];                     // right traces of columns -1 .. TX-1, then the x face fluxes
+  union {
+    struct {
+      double yb[O][TY + 1][TX][4];                 // bottom traces of rows 0 .. TY
+      double xl[O][TY][TX + 1][4];                 // left traces of columns 0 .. TX
+    } tr;
+    union {
+      double nodes[NB][3][TX][4];                  // f1 (first the node values), f2, s
+      LimitLds lim;
+    } wave[TY];
+  } u;
+};
+
+template <int O, int TY, bool HLLC>
+__global__ __launch_bounds__(64 * TY, 4) void dgq_stage_kernel(Geo g, Tab T, const double* __restrict__ in,
+                                                            const double* __restrict__ x, const double* __restrict__ y,
+                                                            const double* __restrict__ gx,
+                                                            const double* __restrict__ gy, Epi e, double* out,
+                                                            Clock* __restrict__ ck) {
+  if (ck && !ck->active) return;
+  using S = StageLds<O, TY>;
+  __shared__ S s;
+  const int nx = g.nx, ny = g.ny;
+  const long long nc = (long long)nx * ny;
+  const double dt = ck ? ck->dt : 0.0;
+  // consecutive tiles on one XCD, whose L2 then holds the halo rows they share
+  const int ntx = (nx + TX - 1) / TX, nt = gridDim.x, per = nt / 8, extra = nt % 8, xcd = blockIdx.x % 8;
+  const int tile = xcd * per + (xcd < extra ? xcd : extra) + blockIdx.x / 8;
+  const int i0 = (tile % ntx) * TX, j0 = (tile / ntx) * TY;
+  const int wl = nx - i0 < TX ? nx - i0 : TX, hl = ny - j0 < TY ? ny - j0 : TY;
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, col = lane >> 2, v = lane & 3;
+  const bool own = col < wl && w < hl;
+  // lanes outside the tile repeat its last cell and store nothing
+  const unsigned c = (unsigned)(i0 + (col < wl ? col : wl - 1) + nx * (j0 + (w < hl ? w : hl - 1)));
+  const unsigned la = 8u * (v + 4u * c);
+
+  double m[O][O];
+  load_modes<O>(in, la, nc, m);
+  if (w < 3) {
+    int hc = 0;
+    bool has;
+    if (w < 2) {                                   // the row below, the row above
+      const int jh = w == 0 ? (j0 > 0 ? j0 - 1 : g.bc == 1 ? ny - 1 : 0)
+                            : (j0 + hl < ny ? j0 + hl : g.bc == 1 ? 0 : ny - 1);
+      has = col < wl;
+      hc = i0 + (has ? col : 0) + nx * jh;
+    } else {                                       // columns left and right
+      const int r = col % TY;
+      const int ih = col < TY ? (i0 > 0 ? i0 - 1 : g.bc == 1 ? nx - 1 : 0)
+                              : (i0 + wl < nx ? i0 + wl : g.bc == 1 ? 0 : nx - 1);
+      has = col < 2 * TY && r < hl;
+      hc = ih + nx * (j0 + (has ? r : 0));
+    }
+    double mh[O][O];
+    load_modes<O>(in, 8u * (v + 4u * hc), nc, mh);
+    if (w < 2) {
+#pragma unroll
+      for (int q = 0; q < O; ++q) {
+        const double lo = trace_y<O>(T, mh, false, q), hi = trace_y<O>(T, mh, true, q);
+        if (has) *(w == 0 ? &s.yt[q][0][col][v] : &s.u.tr.yb[q][hl][col][v]) = w == 0 ? hi : lo;
       }
+    } else {
+      const bool left = col < TY;
+#pragma unroll
+      for (int q = 0; q < O; ++q) {
+        const double lo = trace_x<O>(T, mh, false, q), hi = trace_x<O>(T, mh, true, q);
+        if (has) *(left ? &s.xr[q][col % TY][0][v] : &s.u.tr.xl[q][col % TY][wl][v]) = left ? hi : lo;
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < O; ++q) {
+    const double l = trace_x<O>(T, m, false, q), r = trace_x<O>(T, m, true, q);
+    const double b = trace_y<O>(T, m, false, q), t = trace_y<O>(T, m, true, q);
+    if (own) {
+      s.u.tr.xl[q][w][col][v] = l;
+      s.xr[q][w][col + 1][v] = r;
+      s.u.tr.yb[q][w][col][v] = b;
+      s.yt[q][w + 1][col][v] = t;
+    }
+  }
+  __syncthreads();
+
+  constexpr int NY = O * (TY + 1) * TX, NX = O * TY * (TX + 1);
+#pragma unroll 1
+  for (int k = tid; k < NY + NX; k += 64 * TY) {
+    const bool xdir = k >= NY;
+    const int kx = k - NY;
+    if (xdir ? (kx % (TX + 1) > wl || kx / (TX + 1) % TY >= hl) : (k % TX >= wl || k / TX % (TY + 1) > hl)) continue;
+    double* lo = xdir ? &s.xr[0][0][0][0] + 4 * kx : &s.yt[0][0][0][0] + 4 * k;
+    const double* hi = xdir ? &s.u.tr.xl[0][0][0][0] + 4 * kx : &s.u.tr.yb[0][0][0][0] + 4 * k;
+    double ul[4], ur[4], fl[4], fr[4], f[4];
+    get4(lo, ul);
+    get4(hi, ur);
+    flux_int(g.gamma, ul, xdir ? 0 : 1, fl);
+    flux_int(g.gamma, ur, xdir ? 0 : 1, fr);
+    num_flux<HLLC>(g, ul, ur, fl, fr, xdir ? 1 : 2, f);
+    put4(lo, f);
+  }
+  __syncthreads();
+
+  // f1 P(a,0) and f2 P(b,0) are products with zero: the integrals of the modes
+  // i = 0 (along x) and j = 0 (along y) are 0, or NaN if a flux is not finite
+  constexpr int NB = S::NB;
+  double fv1[O][O], fv2[O][O], sv[O][O], z1 = 0.0, z2 = 0.0;
+#pragma unroll
+  for (int i = 0; i < O; ++i)
+#pragma unroll
+    for (int j = 0; j < O; ++j) fv1[i][j] = fv2[i][j] = sv[i][j] = 0.0;
+  const bool has_s = g.source != 1;
+  double(*nd)[3][TX][4] = s.u.wave[w].nodes;
+#pragma unroll 1
+  for (int a0 = 0; a0 < O; a0 += NB / O) {
+    // this lane's node of the pass (lane 3 of a cell has none for O = 3)
+    const int an = O == 2 ? v >> 1 : a0, bn = O == 2 ? v & 1 : v;
+    double g0 = 0.0, g1 = 0.0;
+    if (g.source == 2 && bn < O) {
+      const unsigned k = c + (unsigned)nc * (an + O * bn);
+      g0 = cell_value(gx, k);
+      g1 = cell_value(gy, k);
+    }
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {                 // get_nodes_from_modes (:544-592)
+      const int a = O == 2 ? k / O : a0, b = k % O;
+      nd[k][0][col][v] = node_value<O>(T, m, a, b);
+    }
+    wave_lds_sync();
+    if (v < NB) {
+      double u[4], f1[4], f2[4], sq[4] = {0.0, 0.0, 0.0, 0.0};
+      get4(nd[v][0][col], u);
+      flux_full(g.gamma, u, f1, f2);
+      if (g.source == 2) {                         // get_source (:1558-1576)
+        double p[4];
+        prim(g.gamma, u, p);
+        sq[1] = p[0] * g0;
+        sq[2] = p[0] * g1;
+        sq[3] = p[0] * (p[1] * g0 + p[2] * g1);
+      } else if (g.source == 3) {                  // get_adv_source (:1579-1596)
+        sq[0] = -1.0 * u[0];
+      }
+      put4(nd[v][0][col], f1);
+      put4(nd[v][1][col], f2);
+      if (has_s) put4(nd[v][2][col], sq);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int a = O == 2 ? k / O : a0, b = k % O;
+      const double f1 = nd[k][0][col][v], f2 = nd[k][1][col][v];
+      z1 = z1 + f1 * 0.0;
+      z2 = z2 + f2 * 0.0;
+#pragma unroll
+      for (int i = 1; i < O; ++i) {
+        const double f1i = f1 * T.P[a][i] * T.wq[a], f2j = times_pw<O>(T, f2, b, i);
+#pragma unroll
+        for (int j = 0; j < O; ++j) {
+          fv1[i][j] = fv1[i][j] + times_l<O>(T, f1i, b, j) * weight<O>(T, b);
+          fv2[j][i] = fv2[j][i] + times_row(T, f2j, a, j) * T.wq[a];
+        }
+      }
+      if (has_s) {
+        const double sq = nd[k][2][col][v];
+#pragma unroll
+        for (int i = 0; i < O; ++i) {
+          const double si = times_row(T, sq, a, i) * T.wq[a];
+#pragma unroll
+          for (int j = 0; j < O; ++j) sv[i][j] = sv[i][j] + times_l<O>(T, si, b, j) * weight<O>(T, b);
+        }
+      }
+    }
+    wave_lds_sync();
+  }
+
+  // :1455-1462 (oneoverdx for the y terms too), the volume, x edge and y edge
+  // terms one after the other so that few values are live at a time
+  const double odx = g.odx;
+  double d[O][O];
+#pragma unroll
+  for (int i = 0; i < O; ++i)
+#pragma unroll
+    for (int j = 0; j < O; ++j) d[i][j] = odx * (i == 0 ? z1 : fv1[i][j]) + odx * (j == 0 ? z2 : fv2[i][j]);
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    double fl[O], fr[O];
+#pragma unroll
+    for (int q = 0; q < O; ++q) {
+      fl[q] = s.xr[q][w][col][v];
+      fr[q] = s.xr[q][w][col + 1][v];
+    }
+#pragma unroll
+    for (int i = 0; i < O; ++i)
+#pragma unroll
+      for (int j = 0; j < O; ++j) {
+        double e1 = 0.0, e2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < O; ++q) {              // :1377-1386
+          e1 = e1 + times_l<O>(T, times_edge(T, fr[q], true, i), q, j) * weight<O>(T, q);
+          e2 = e2 + times_l<O>(T, times_edge(T, fl[q], false, i), q, j) * weight<O>(T, q);
+        }
+        d[i][j] = d[i][j] - odx * (e1 - e2);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  {
+    double gb[O], gt[O];
+#pragma unroll
+    for (int q = 0; q < O; ++q) {
+      gb[q] = s.yt[q][w][col][v];
+      gt[q] = s.yt[q][w + 1][col][v];
+    }
+#pragma unroll
+    for (int j = 0; j < O; ++j)
+#pragma unroll
+      for (int i = 0; i < O; ++i) {
+        double e3 = 0.0, e4 = 0.0;
+#pragma unroll
+        for (int q = 0; q < O; ++q) {              // :1391-1408
+          e3 = e3 + times_l<O>(T, times_edge(T, gt[q], true, j), q, i) * weight<O>(T, q);
+          e4 = e4 + times_l<O>(T, times_edge(T, gb[q], false, j), q, i) * weight<O>(T, q);
+        }
+        d[i][j] = (d[i][j] - odx * (e3 - e4)) / 2. + sv[i][j] / 4.;
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (g.ninit == 12) {                             // special_boundary_conditions (:1481-1514)
+#pragma unroll
+    for (int i = 0; i < O; ++i)
+#pragma unroll
+      for (int j = 0; j < O; ++j) {
+        const double xd = cell_value(x + nc * (i + O * j), c) - g.boxlen_x / 2.;
+        const double yd = cell_value(y + nc * (i + O * j), c) - g.boxlen_y / 2.;
+        if (sqrt(xd * xd + yd * yd) > 2.0) d[i][j] = 0.0;
+      }
+  }
+
+  // w5 needs L and its leading terms once the result is limited: they wait in
+  // their lane's elements of out and w5, which no other lane reads, and not in
+  // registers
+  if (own && e.w5) {
+#pragma unroll
+    for (int j = 0; j < O; ++j)
+#pragma unroll
+      for (int i = 0; i < O; ++i) {
+        mode<O>(e.w5, la, nc, i, j) =
+            e.b0 * mode<O>(e.X, la, nc, i, j) + e.b1 * mode<O>(e.Y, la, nc, i, j) + e.bm * m[i][j];
+        mode<O>(out, la, nc, i, j) = d[i][j];
+      }
+  }
+  if (e.combine) {
+    if (e.X) {
+      const double* X = e.X;
+#pragma unroll
+      for (int j = 0; j < O; ++j)
+#pragma unroll
+        for (int i = 0; i < O; ++i) {
+          const double ax = e.a * mode<O>(X, la, nc, i, j);
+          m[i][j] = e.own ? ax + e.am * m[i][j] : ax;
+        }
+    } else {
+#pragma unroll
+      for (int j = 0; j < O; ++j)
+#pragma unroll
+        for (int i = 0; i < O; ++i) m[i][j] = e.am * m[i][j];
+    }
+#pragma unroll
+    for (int j = 0; j < O; ++j)
+#pragma unroll
+      for (int i = 0; i < O; ++i) d[i][j] = m[i][j] + e.cdt * dt * d[i][j];
+  }
+  if (e.limit) limit_cells<O>(g, T, s.u.wave[w].lim, d);
+  if (own && e.w5) {
+#pragma unroll
+    for (int j = 0; j < O; ++j)
+#pragma unroll
+      for (int i = 0; i < O; ++i) {
+        const double part = mode<O>(e.w5, la, nc, i, j), l = mode<O>(out, la, nc, i, j);
+        mode<O>(e.w5, la, nc, i, j) = part + e.b4 * d[i][j] + e.c5 * dt * l;
+      }
+  }
+  if (own) {
+#pragma unroll
+    for (int j = 0; j < O; ++j)
+#pragma unroll
+      for (int i = 0; i < O; ++i) mode<O>(out, la, nc, i, j) = d[i][j];
+  }
+  if (e.tick && blockIdx.x == 0 && tid == 0) {     // t = t + dt (:749); no block reads these
+    ck->t = ck->t + dt;
+    ck->dt_last = dt;
+    ck->steps += 1;
+  }
+}
+
+// the state of 'DEB', whose stage reads the neighbours of what it replaces
+__global__ __launch_bounds__(256) void dgq_copy_kernel(long long n, const double* __restrict__ src,
+                                                       double* __restrict__ dst, const Clock* __restrict__ ck) {
+  if (!ck->active) return;
+  for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < n; k += (long long)gridDim.x * 256) dst[k] = src[k];
 }
 
 // get_nodes_from_modes / get_modes_from_nodes (:497-592) per cell, in the
@@ -766,7 +965,7 @@ __device__ __forceinline__ bool speed_runs(const Clock* ck, double t_end) {
 
 // the pairs of every block combined (each thread of the block strides over
 // them, then the block reduces): S and k* (-1 when no speed reached S >= 0)
-__device__ void combine_pairs(const double* __restrict__ part, int nblk, double& S, long long& ks) {
+__device__ void combine_pairs(const double* part, int nblk, double& S, long long& ks) {
   __shared__ double sd[SPEED_THREADS / 64];
   __shared__ long long sk[SPEED_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -784,10 +983,7 @@ __device__ void combine_pairs(const double* __restrict__ part, int nblk, double&
   __syncthreads();
 }
 
-__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_pairs_kernel(Geo g, const double* __restrict__ u,
-                                                                       double* __restrict__ part,
-                                                                       const Clock* __restrict__ ck, double t_end) {
-  if (!speed_runs(ck, t_end)) return;
+__device__ void speed_pairs(const Geo& g, const double* __restrict__ u, double* part) {
   __shared__ double sd[SPEED_THREADS / 64];
   __shared__ long long sk[SPEED_THREADS / 64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -813,10 +1009,7 @@ __global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_pairs_kernel(Geo g, c
   }
 }
 
-__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_csmin_kernel(Geo g, const double* __restrict__ u,
-                                                                       double* __restrict__ part,
-                                                                       const Clock* __restrict__ ck, double t_end) {
-  if (!speed_runs(ck, t_end)) return;
+__device__ void speed_csmin(const Geo& g, const double* __restrict__ u, double* part) {
   __shared__ double sd[SPEED_THREADS / 64];
   double S;
   long long ks;
@@ -844,14 +1037,8 @@ __global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_csmin_kernel(Geo g, c
   }
 }
 
-__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_final_kernel(Geo g, const double* __restrict__ u,
-                                                                       const double* __restrict__ part, int nblk,
-                                                                       double* __restrict__ res,
-                                                                       Clock* __restrict__ ck, double t_end) {
-  if (!speed_runs(ck, t_end)) {
-    if (threadIdx.x == 0) ck->active = 0;
-    return;
-  }
+__device__ void speed_final(const Geo& g, const double* __restrict__ u, const double* part, int nblk,
+                            double* __restrict__ res, Clock* __restrict__ ck, double t_end) {
   double S;
   long long ks;
   combine_pairs(part, nblk, S, ks);
@@ -895,12 +1082,34 @@ __global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_final_kernel(Geo g, c
   }
 }
 
-// t = t + dt (:749), after the step
-__global__ void dgq_tick_kernel(Clock* __restrict__ ck) {
-  if (threadIdx.x != 0 || !ck->active) return;
-  ck->t = ck->t + ck->dt;
-  ck->dt_last = ck->dt;
-  ck->steps += 1;
+__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_pairs_kernel(Geo g, const double* __restrict__ u,
+                                                                       double* __restrict__ part,
+                                                                       const Clock* __restrict__ ck, double t_end) {
+  if (speed_runs(ck, t_end)) speed_pairs(g, u, part);
+}
+
+__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_csmin_kernel(Geo g, const double* __restrict__ u,
+                                                                       double* __restrict__ part,
+                                                                       const Clock* __restrict__ ck, double t_end) {
+  if (speed_runs(ck, t_end)) speed_csmin(g, u, part);
+}
+
+// the last of the three launches, or (alone: one block, small grids) all three
+__global__ __launch_bounds__(SPEED_THREADS) void dgq_speed_final_kernel(Geo g, const double* __restrict__ u,
+                                                                       double* part, int nblk, bool alone,
+                                                                       double* __restrict__ res,
+                                                                       Clock* __restrict__ ck, double t_end) {
+  if (!speed_runs(ck, t_end)) {
+    if (threadIdx.x == 0) ck->active = 0;
+    return;
+  }
+  if (alone) {
+    speed_pairs(g, u, part);
+    __syncthreads();
+    speed_csmin(g, u, part);
+    __syncthreads();
+  }
+  speed_final(g, u, part, nblk, res, ck, t_end);
 }
 
 // compute_error (:23-89) per cell, then a fixed-order sum of the block
@@ -973,13 +1182,13 @@ struct fvwb_dgq {
   hipStream_t stream = nullptr;
   long long nc = 0, ns = 0;                  // cells, doubles per state
   double* du = nullptr;                      // resident state
-  double* w[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};   // stage states; w[5] holds L(w3)
+  double* w[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};   // stage states
   double* s_in = nullptr;                    // drop-in staging
   double* s_out = nullptr;
   double *x = nullptr, *y = nullptr;         // resident coordinates
   double *xi = nullptr, *yi = nullptr;       // drop-in coordinates
-  double* tr = nullptr;                      // traces and their fluxes
-  double *F = nullptr, *G = nullptr;
+  double *gx = nullptr, *gy = nullptr;       // grad_phi at the resident coordinates (source 2)
+  double *gxi = nullptr, *gyi = nullptr;     // and at the drop-in's
   double* res = nullptr;                     // small results
   double* part = nullptr;                    // error partials
   Clock* clk = nullptr;
@@ -1031,8 +1240,8 @@ extern "C" int fvwb_dgq_params_reference(fvwb_dgq_params* p) {
 extern "C" int fvwb_dgq_destroy(fvwb_dgq_handle h) {
   if (!h) return FVWB_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
-  void* ps[] = {h->du, h->w[0], h->w[1], h->w[2], h->w[3], h->w[4], h->w[5], h->s_in, h->s_out, h->x, h->y, h->xi,
-                h->yi, h->tr, h->F, h->G, h->res, h->part, h->clk};
+  void* ps[] = {h->du, h->w[0], h->w[1], h->w[2], h->w[3], h->w[4], h->s_in, h->s_out, h->x, h->y, h->xi, h->yi,
+                h->gx, h->gy, h->gxi, h->gyi, h->res, h->part, h->clk};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1048,14 +1257,21 @@ static long long err_blocks(long long nc) { return (nc + ERR_THREADS - 1) / ERR_
 static int speed_blocks(long long nc) {
   return (int)std::max(1LL, std::min<long long>((nc + SPEED_THREADS - 1) / SPEED_THREADS, SPEED_MAX_BLOCKS));
 }
+// up to four cells per thread of one block the one launch is the faster form:
+// 45 against 52 us per 'RK4' step at 16^2, 76 against 78 at 32^2; at 64^2 the
+// block is the bound (38 against 31 us per 'EQL' step)
+static constexpr long long SPEED_ALONE_CELLS = 4 * SPEED_THREADS;
 static void launch_speed(fvwb_dgq* h, const double* u, double* res, Clock* ck, double t_end) {
-  const int nb = speed_blocks(h->nc);
-  hipLaunchKernelGGL(dgq_speed_pairs_kernel, dim3(nb), dim3(SPEED_THREADS), 0, h->stream, h->g, u, h->part,
-                     (const Clock*)ck, t_end);
-  hipLaunchKernelGGL(dgq_speed_csmin_kernel, dim3(nb), dim3(SPEED_THREADS), 0, h->stream, h->g, u, h->part,
-                     (const Clock*)ck, t_end);
-  hipLaunchKernelGGL(dgq_speed_final_kernel, dim3(1), dim3(SPEED_THREADS), 0, h->stream, h->g, u,
-                     (const double*)h->part, nb, res, ck, t_end);
+  const bool alone = h->nc <= SPEED_ALONE_CELLS;
+  const int nb = alone ? 1 : speed_blocks(h->nc);
+  if (!alone) {
+    hipLaunchKernelGGL(dgq_speed_pairs_kernel, dim3(nb), dim3(SPEED_THREADS), 0, h->stream, h->g, u, h->part,
+                       (const Clock*)ck, t_end);
+    hipLaunchKernelGGL(dgq_speed_csmin_kernel, dim3(nb), dim3(SPEED_THREADS), 0, h->stream, h->g, u, h->part,
+                       (const Clock*)ck, t_end);
+  }
+  hipLaunchKernelGGL(dgq_speed_final_kernel, dim3(1), dim3(SPEED_THREADS), 0, h->stream, h->g, u, h->part, nb, alone,
+                     res, ck, t_end);
 }
 
 extern "C" int fvwb_dgq_create(fvwb_dgq_handle* out, const fvwb_dgq_params* p) {
@@ -1088,18 +1304,16 @@ extern "C" int fvwb_dgq_create(fvwb_dgq_handle* out, const fvwb_dgq_params* p) {
   h->nc = (long long)p->nx * p->ny;
   h->ns = 4 * h->nc * o * o;
   const size_t sb = sizeof(double) * (size_t)h->ns, cb = sizeof(double) * (size_t)(h->nc * o * o);
-  const size_t trb = sizeof(double) * (size_t)(32LL * o * h->nc);
-  const size_t fb = sizeof(double) * (size_t)(4LL * o * (p->nx + 1) * p->ny);
-  const size_t gb = sizeof(double) * (size_t)(4LL * o * p->nx * (p->ny + 1));
   bool ok = hipStreamCreate(&h->stream) == hipSuccess && hipMalloc(&h->du, sb) == hipSuccess &&
             hipMalloc(&h->s_in, sb) == hipSuccess && hipMalloc(&h->s_out, sb) == hipSuccess &&
             hipMalloc(&h->x, cb) == hipSuccess && hipMalloc(&h->y, cb) == hipSuccess &&
             hipMalloc(&h->xi, cb) == hipSuccess && hipMalloc(&h->yi, cb) == hipSuccess &&
-            hipMalloc(&h->tr, trb) == hipSuccess && hipMalloc(&h->F, fb) == hipSuccess &&
-            hipMalloc(&h->G, gb) == hipSuccess && hipMalloc(&h->res, 16 * sizeof(double)) == hipSuccess &&
+            hipMalloc(&h->res, 16 * sizeof(double)) == hipSuccess &&
             hipMalloc(&h->part, sizeof(double) * 12 * (size_t)err_blocks(h->nc)) == hipSuccess &&
             hipMalloc(&h->clk, sizeof(Clock)) == hipSuccess;
-  for (int k = 0; ok && k < 6; ++k) ok = hipMalloc(&h->w[k], sb) == hipSuccess;
+  for (int k = 0; ok && k < 5; ++k) ok = hipMalloc(&h->w[k], sb) == hipSuccess;
+  if (p->source == 2)
+    for (double** q : {&h->gx, &h->gy, &h->gxi, &h->gyi}) ok = ok && hipMalloc(q, cb) == hipSuccess;
   if (!ok) {
     fvwb_dgq_destroy(h);
     return failq(nullptr, FVWB_ERR_OOM, "device allocation failed");
@@ -1109,36 +1323,45 @@ extern "C" int fvwb_dgq_create(fvwb_dgq_handle* out, const fvwb_dgq_params* p) {
 }
 
 static dim3 cells_grid(const fvwb_dgq* h) { return dim3((unsigned)((h->nc + 255) / 256)); }
-static dim3 cell_grid(const fvwb_dgq* h) { return dim3((unsigned)((h->nc + CELL_THREADS - 1) / CELL_THREADS)); }
-static dim3 finish_grid(const fvwb_dgq* h) { return dim3((unsigned)std::min<long long>((h->ns + 255) / 256, 8192)); }
 
-// compute_update of `in` into `out` with the stage combination e (nterms = 0:
-// dudt itself); the clock gates and provides dt in the resident loop.
-static int residual(fvwb_dgq* h, const double* in, const double* x, const double* y, const Epi& e, double* out,
-                    const Clock* ck) {
-  const long long nf = (long long)(h->p.nx + 1) * h->p.ny * h->p.order + (long long)h->p.nx * (h->p.ny + 1) * h->p.order;
-  const dim3 fg((unsigned)((nf + 255) / 256));
-  if (h->p.order == 2) {
-    hipLaunchKernelGGL(dgq_trace_kernel<2>, cells_grid(h), dim3(256), 0, h->stream, h->g, h->T, in, h->tr, ck);
-    hipLaunchKernelGGL(dgq_face_kernel<2>, fg, dim3(256), 0, h->stream, h->g, h->tr, h->F, h->G, ck);
-    hipLaunchKernelGGL(dgq_cell_kernel<2>, cell_grid(h), dim3(CELL_THREADS), 0, h->stream, h->g, h->T, in, x, y,
-                       h->F, h->G, e, out, ck);
-  } else {
-    hipLaunchKernelGGL(dgq_trace_kernel<3>, cells_grid(h), dim3(256), 0, h->stream, h->g, h->T, in, h->tr, ck);
-    hipLaunchKernelGGL(dgq_face_kernel<3>, fg, dim3(256), 0, h->stream, h->g, h->tr, h->F, h->G, ck);
-    hipLaunchKernelGGL(dgq_cell_kernel<3>, cell_grid(h), dim3(CELL_THREADS), 0, h->stream, h->g, h->T, in, x, y,
-                       h->F, h->G, e, out, ck);
-  }
+// the fields of the residual beside the state: coordinates and grad_phi
+struct Coords {
+  const double *x, *y, *gx, *gy;
+};
+
+static int gradients(fvwb_dgq* h, const double* x, const double* y, double* gx, double* gy) {
+  if (h->p.source != 2) return FVWB_OK;
+  const long long n = h->nc * h->p.order * h->p.order;
+  hipLaunchKernelGGL(dgq_grad_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->g.gpc, n, x, y, gx,
+                     gy);
   HIPQ(h, hipGetLastError());
   return FVWB_OK;
 }
 
-static int limit(fvwb_dgq* h, double* u, const Clock* ck) {
+template <int O, int TY>
+static void launch_stage(fvwb_dgq* h, const double* in, const Coords& k, const Epi& e, double* out, Clock* ck) {
+  const unsigned nt = (unsigned)(((h->p.nx + TX - 1) / TX) * ((h->p.ny + TY - 1) / TY));
+  auto* kernel = h->p.flux_type == FVWB_DGQ_FLUX_HLLC ? dgq_stage_kernel<O, TY, true> : dgq_stage_kernel<O, TY, false>;
+  hipLaunchKernelGGL(kernel, dim3(nt), dim3(64 * TY), 0, h->stream, h->g, h->T, in, k.x, k.y, k.gx, k.gy, e, out, ck);
+}
+
+// compute_update of `in` into `out` with the stage combination e (combine = 0:
+// dudt itself); the clock gates and provides dt in the resident loop.  `out`
+// may be e.X but not `in`, whose neighbours other tiles read.
+static int stage(fvwb_dgq* h, const double* in, const Coords& k, const Epi& e, double* out, Clock* ck) {
+  if (h->p.order == 2) launch_stage<2, 4>(h, in, k, e, out, ck);
+  else launch_stage<3, 4>(h, in, k, e, out, ck);
+  HIPQ(h, hipGetLastError());
+  return FVWB_OK;
+}
+
+static int limit(fvwb_dgq* h, double* u) {
   if (!h->p.use_limiter) return FVWB_OK;
+  const dim3 grid((unsigned)((h->nc + 4 * TX - 1) / (4 * TX)));
   if (h->p.order == 2)
-    hipLaunchKernelGGL(dgq_limit_kernel<2>, cells_grid(h), dim3(256), 0, h->stream, h->g, h->T, u, ck);
+    hipLaunchKernelGGL(dgq_limit_kernel<2>, grid, dim3(256), 0, h->stream, h->g, h->T, u);
   else
-    hipLaunchKernelGGL(dgq_limit_kernel<3>, cells_grid(h), dim3(256), 0, h->stream, h->g, h->T, u, ck);
+    hipLaunchKernelGGL(dgq_limit_kernel<3>, grid, dim3(256), 0, h->stream, h->g, h->T, u);
   HIPQ(h, hipGetLastError());
   return FVWB_OK;
 }
@@ -1176,9 +1399,8 @@ extern "C" int fvwb_dgq_compute_update(fvwb_dgq_handle h, const double* delta_u,
   HIPQ(h, hipMemcpyAsync(h->s_in, delta_u, state_bytes(h), hipMemcpyHostToDevice, h->stream));
   HIPQ(h, hipMemcpyAsync(h->xi, x, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
   HIPQ(h, hipMemcpyAsync(h->yi, y, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
-  Epi e{};
-  int rc = residual(h, h->s_in, h->xi, h->yi, e, h->s_out, nullptr);
-  if (rc) return rc;
+  int rc = gradients(h, h->xi, h->yi, h->gxi, h->gyi);
+  if (rc || (rc = stage(h, h->s_in, Coords{h->xi, h->yi, h->gxi, h->gyi}, Epi{}, h->s_out, nullptr))) return rc;
   HIPQ(h, hipMemcpyAsync(dudt, h->s_out, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
@@ -1203,7 +1425,7 @@ extern "C" int fvwb_dgq_compute_max_speed(fvwb_dgq_handle h, const double* u, do
 extern "C" int fvwb_dgq_apply_limiter(fvwb_dgq_handle h, double* u) {
   if (!h || !u) return failq(h, FVWB_ERR_ARG, "NULL argument");
   HIPQ(h, hipMemcpyAsync(h->s_in, u, state_bytes(h), hipMemcpyHostToDevice, h->stream));
-  int rc = limit(h, h->s_in, nullptr);
+  int rc = limit(h, h->s_in);
   if (rc) return rc;
   HIPQ(h, hipMemcpyAsync(u, h->s_in, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
@@ -1235,6 +1457,8 @@ extern "C" int fvwb_dgq_upload(fvwb_dgq_handle h, const double* delta_u, const d
   HIPQ(h, hipMemcpyAsync(h->x, x, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
   HIPQ(h, hipMemcpyAsync(h->y, y, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
   HIPQ(h, hipMemcpyAsync(h->clk, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
+  int rc = gradients(h, h->x, h->y, h->gx, h->gy);
+  if (rc) return rc;
   HIPQ(h, hipStreamSynchronize(h->stream));
   h->loaded = true;
   return FVWB_OK;
@@ -1256,14 +1480,17 @@ static const float kSS4[16] = {0.39175222700392f, 0.44437049406734f, 0.555629505
                                0.82192004589227f, 0.54497475021237f, 0.00683325884039f, 0.51723167208978f,
                                0.12759831133288f, 0.34833675773694f, 0.08460416338212f, 0.22600748319395f};
 
-static Epi epi(std::initializer_list<std::pair<double, const double*>> terms, double cdt) {
+// a X + am in + cdt dt L (X = nullptr, or am = 0: without that term)
+static Epi epi(const fvwb_dgq* h, double a, const double* X, double am, double cdt, bool last = false) {
   Epi e{};
-  for (const auto& t : terms) {
-    e.a[e.nterms] = t.first;
-    e.X[e.nterms] = t.second;
-    ++e.nterms;
-  }
+  e.X = X;
+  e.a = a;
+  e.am = am;
   e.cdt = cdt;
+  e.combine = 1;
+  e.own = am != 0.0;
+  e.limit = h->p.use_limiter;
+  e.tick = last;
   return e;
 }
 
@@ -1272,41 +1499,37 @@ static Epi epi(std::initializer_list<std::pair<double, const double*>> terms, do
 static int step(fvwb_dgq* h, double t_end) {
   Clock* ck = h->clk;
   double* du = h->du;
-  double *w1 = h->w[0], *w2 = h->w[1], *w3 = h->w[2], *w4 = h->w[3], *w5 = h->w[4], *l3 = h->w[5];
+  double *w1 = h->w[0], *w2 = h->w[1], *w3 = h->w[2], *w4 = h->w[3], *w5 = h->w[4];
   launch_speed(h, du, nullptr, ck, t_end);
   HIPQ(h, hipGetLastError());
   int rc = 0;
-  const double *x = h->x, *y = h->y;
+  const Coords k{h->x, h->y, h->gx, h->gy};
   if (h->p.solver == FVWB_DGQ_SOLVER_EQL) {        // :672-681
-    if ((rc = residual(h, du, x, y, epi({{1.0, du}}, 1.0), w1, ck)) || (rc = limit(h, w1, ck))) return rc;
-    if ((rc = residual(h, w1, x, y, epi({{0.5, du}, {0.5, w1}}, 0.5), du, ck)) || (rc = limit(h, du, ck))) return rc;
-  } else if (h->p.solver == FVWB_DGQ_SOLVER_DEB) { // :737-747: w1 = du + dt L(du), limited, becomes du
-    if ((rc = residual(h, du, x, y, epi({{1.0, du}}, 1.0), du, ck)) || (rc = limit(h, du, ck))) return rc;
-  } else {                                          // 'RK4' / 'SS4'
-    const float* cf = h->p.solver == FVWB_DGQ_SOLVER_SS4 ? kSS4 : kRK4;
-    double c[16];
-    for (int k = 0; k < 16; ++k) c[k] = (double)cf[k];
-    if ((rc = residual(h, du, x, y, epi({{1.0, du}}, c[0]), w1, ck)) || (rc = limit(h, w1, ck))) return rc;
-    if ((rc = residual(h, w1, x, y, epi({{c[1], du}, {c[2], w1}}, c[3]), w2, ck)) || (rc = limit(h, w2, ck))) return rc;
-    if ((rc = residual(h, w2, x, y, epi({{c[4], du}, {c[5], w2}}, c[6]), w3, ck)) || (rc = limit(h, w3, ck))) return rc;
-    // w4 = c7 u + c8 w3 + c9 dt L(w3).  The reference evaluates L(w3) once more
-    // (:700, :723) for w5 = c10 u + c11 w2 + c12 w3 + c13 w4 + c14 dt L(w3),
-    // with w4 limited; here the first evaluation also keeps L(w3) and the sum
-    // of w5's first three terms, and w5 is finished once w4 is limited.
-    Epi e4 = epi({{c[7], du}, {c[8], w3}}, c[9]);
-    e4.Y[0] = du; e4.Y[1] = w2; e4.Y[2] = w3;
-    e4.b[0] = c[10]; e4.b[1] = c[11]; e4.b[2] = c[12];
-    e4.npart = 3; e4.part = w5; e4.lval = l3;
-    if ((rc = residual(h, w3, x, y, e4, w4, ck)) || (rc = limit(h, w4, ck))) return rc;
-    hipLaunchKernelGGL(dgq_finish_kernel, finish_grid(h), dim3(256), 0, h->stream, h->ns, (const double*)w5, c[13],
-                       (const double*)w4, c[14], (const double*)l3, w5, (const Clock*)ck);
-    HIPQ(h, hipGetLastError());
-    // then L(w4) for the new state
-    if ((rc = residual(h, w4, x, y, epi({{1.0, w5}}, c[15]), du, ck)) || (rc = limit(h, du, ck))) return rc;
+    if ((rc = stage(h, du, k, epi(h, 0.0, nullptr, 1.0, 1.0), w1, ck))) return rc;
+    return stage(h, w1, k, epi(h, 0.5, du, 0.5, 0.5, true), du, ck);
   }
-  hipLaunchKernelGGL(dgq_tick_kernel, dim3(1), dim3(64), 0, h->stream, ck);
-  HIPQ(h, hipGetLastError());
-  return FVWB_OK;
+  if (h->p.solver == FVWB_DGQ_SOLVER_DEB) {        // :737-747: w1 = du + dt L(du), limited, becomes du
+    if ((rc = stage(h, du, k, epi(h, 0.0, nullptr, 1.0, 1.0, true), w1, ck))) return rc;
+    hipLaunchKernelGGL(dgq_copy_kernel, dim3((unsigned)std::min<long long>((h->ns + 255) / 256, 8192)), dim3(256), 0,
+                       h->stream, h->ns, (const double*)w1, du, (const Clock*)ck);
+    HIPQ(h, hipGetLastError());
+    return FVWB_OK;
+  }
+  const float* cf = h->p.solver == FVWB_DGQ_SOLVER_SS4 ? kSS4 : kRK4;   // 'RK4' / 'SS4'
+  double c[16];
+  for (int q = 0; q < 16; ++q) c[q] = (double)cf[q];
+  if ((rc = stage(h, du, k, epi(h, 0.0, nullptr, 1.0, c[0]), w1, ck))) return rc;
+  if ((rc = stage(h, w1, k, epi(h, c[1], du, c[2], c[3]), w2, ck))) return rc;
+  if ((rc = stage(h, w2, k, epi(h, c[4], du, c[5], c[6]), w3, ck))) return rc;
+  // w4 = c7 u + c8 w3 + c9 dt L(w3), and with w4 limited
+  // w5 = c10 u + c11 w2 + c12 w3 + c13 w4 + c14 dt L(w3)
+  Epi e4 = epi(h, c[7], du, c[8], c[9]);
+  e4.w5 = w5;
+  e4.Y = w2;
+  e4.b0 = c[10]; e4.b1 = c[11]; e4.bm = c[12]; e4.b4 = c[13]; e4.c5 = c[14];
+  if ((rc = stage(h, w3, k, e4, w4, ck))) return rc;
+  // then L(w4) for the new state
+  return stage(h, w4, k, epi(h, 1.0, w5, 0.0, c[15], true), du, ck);
 }
 
 static constexpr int32_t kGroupQ = 32;

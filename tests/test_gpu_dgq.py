@@ -119,6 +119,44 @@ def test_larger_grids_equal_oracle(order, kw):
         np.testing.assert_array_equal(s.download(), out)
 
 
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 34, 66])
+@pytest.mark.parametrize("order", [2, 3])
+def test_tile_edges_and_limited_states(n, order):
+    """Grids that end inside, at and just past the stage kernel's 16 x 4 tiles
+    and either side of the one-launch speed reduction (64^2 cells), over every
+    solver, flux, boundary and source; the limiter on a state whose densities
+    and pressures it has to scale, bit for bit."""
+    k = 2 * n + order
+    kw = dict(flux_type=(n + order) % 4, source=1 + k % 3, grad_phi_case=1 + k % 2, bc=1 + k // 2 % 3, solver=n % 4)
+    say(f"case: dgq tile edges {n}x{n} order {order} {kw}")
+    op = po.make_dgq_params(n, order=order, **kw)
+    x, y = po.dgq_coords(op)
+    rng = np.random.default_rng(k)
+    du = np.zeros((4, n, n, order, order), order="F")
+    du[:, :, :, 0, 0] = np.array([1.0, 0.1, -0.2, 2.5])[:, None, None] + 0.05 * rng.standard_normal((4, n, n))
+    du[:, :, :, 1:, :] = 0.01 * rng.standard_normal(du[:, :, :, 1:, :].shape)
+    du[:, :, :, :, 1:] += 0.01 * rng.standard_normal(du[:, :, :, :, 1:].shape)
+    hard = np.asfortranarray(du.copy())
+    hard[:, : (n + 1) // 2, :, 1:, :] *= 60.0
+    hard[:2, n // 2 :, :, 0, 1:] *= 40.0
+    with fvwb.SolverDGQ(gparams(n, dict(order=order, **kw))) as s:
+        limited = s.apply_limiter(hard)
+        np.testing.assert_array_equal(limited, po.refdg_limiter(op, hard))
+        for d in (du, limited):
+            np.testing.assert_array_equal(s.compute_update(d, x, y), po.refdg_update(op, d, x, y))
+            mean = np.asfortranarray(d[:, :, :, 0, 0])
+            np.testing.assert_array_equal(np.array(s.compute_max_speed(mean)), po.refdg_max_speed(op, mean))
+        s.upload(du, x, y)
+        s.advance(2)
+        out, t, m, _ = po.refdg_evolve(op, du, x, y, float("inf"), max_steps=2)
+        assert s.time()[2] == m == 2 and s.time()[0] == t
+        np.testing.assert_array_equal(s.download(), out)
+        s.advance(4, t_end=1.01 * t)                   # the queued steps past t_end leave the state as it is
+        out, t, m, _ = po.refdg_evolve(op, out, x, y, 1.01 * t, max_steps=4, t0=t)
+        assert s.time()[2] == 2 + m == 3 and s.time()[0] == t
+        np.testing.assert_array_equal(s.download(), out)
+
+
 def test_advance_before_upload_and_bad_shapes():
     with fvwb.SolverDGQ(fvwb.reference_params_dgq()) as s:
         with pytest.raises(fvwb.FvwbError) as e:
