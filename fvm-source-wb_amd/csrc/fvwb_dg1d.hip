@@ -370,6 +370,271 @@ __global__ __launch_bounds__(256) void dg1d_run_kernel(Geometry G, Tables T, Run
   }
 }
 
+// The same loop with everything in one workgroup's LDS, for grids that fit
+// (lds_doubles below).  A stage is two passes with a barrier after each: faces
+// and Gauss points first, each evaluated once and all at the same time (a
+// pair of lanes per face, a thread per point, and in a step's first stage one per cell for
+// the wave speed, whose maximum the second pass needs), then one (mode,
+// variable, cell) per thread: integrals and the stage's line.  The stage input
+// is in LDS, a thread's own U^n and w2 in registers, and the equilibrium's
+// integrals, the same in every stage, are formed once per launch.
+//
+// Bound by the latency of one face's chain of exactly rounded divisions and
+// square roots: 11.6 us per step at 128 cells and three
+// modes against 29 in the other form (one thread per cell and all of its faces,
+// points and modes, in device memory), 17 against 33 at 200 cells, 25 against
+// 60 at 300, 43 against 65 at 480.  With one thread per face, both of its sides
+// one after the other: 13.4 at 128.
+struct Lds {
+  double *st, *fq, *ue, *sq, *px, *F, *uf, *phq, *dphq, *plr, *red;
+};
+__host__ __device__ inline size_t lds_doubles(int n, size_t nx) {
+  return (size_t)12 * n * nx + 6 * (nx + 1) + 2 * n * n + 2 * n + 16;
+}
+template <int N>
+__device__ inline Lds lds_layout(double* p, int nx) {
+  Lds s;
+  s.st = p;  p += 3 * N * nx;            // the stage's input, (3 i + v) nx + c
+  s.fq = p;  p += 3 * N * nx;            // flux at the Gauss points, (3 j + v) nx + c
+  s.ue = p;  p += 3 * N * nx;            // equilibrium there
+  s.sq = p;  p += 2 * N * nx;            // momentum and energy source, (2 j + v - 1) nx + c
+  s.px = p;  p += N * nx;                // phi_q at the first Gauss point's x, q nx + c
+  s.F = p;   p += 3 * (nx + 1);          // face fluxes, v (nx + 1) + f
+  s.uf = p;  p += 3 * (nx + 1);          // equilibrium at the faces
+  s.phq = p; p += N * N;
+  s.dphq = p; p += N * N;
+  s.plr = p; p += 2 * N;
+  s.red = p;                             // a maximum per wave
+  return s;
+}
+
+// face_flux by a pair of lanes, the even one with the left state and the odd one
+// with the right: each forms its own side's primitives, sound speed and, for
+// HLLC, the state that side would give, and `mine` tells which of the two holds
+// the flux.  The operations are face_flux's on the same values.
+__device__ inline void pair_flux(double gamma, int riemann, bool right, const double u[3], double f[3], bool& mine) {
+  if (riemann != FVWB_DG1D_RIEMANN_HLLC) {
+    fv1d::pair_llflux(gamma, right, u, f);
+    mine = !right;
+    return;
+  }
+  using fv1d::other;
+  double w[3];
+  fv1d::primitive(gamma, u, w);
+  const double c = sqrt(gamma * fmax(w[2], 1e-10) / fmax(w[0], 1e-10));
+  const double cm = fmax(c, other(c)), w1o = other(w[1]);
+  const double s = right ? fmax(w1o, w[1]) + cm : fmin(w[1], w1o) - cm;
+  const double k = s - w[1], d = w[0] * (right ? k : -k);
+  const double dn = other(d), w2o = other(w[2]), so = other(s);
+  const double dl = right ? dn : d, dr = right ? d : dn;
+  const double vl = right ? w1o : w[1], vr = right ? w[1] : w1o;
+  const double pl = right ? w2o : w[2], pr = right ? w[2] : w2o;
+  const double us = (dr * vr + dl * vl + (pl - pr)) / (dl + dr);
+  const double ps = (dr * pl + dl * pr + dl * dr * (vl - vr)) / (dl + dr);
+  double g0 = w[0], g1 = w[1], g2 = w[2], e = u[2];
+  if (right ? s > 0.0 : !(s > 0.0)) {
+    g0 = w[0] * k / (s - us);
+    g1 = us;
+    g2 = ps;
+    e = (k * u[2] - w[2] * w[1] + ps * us) / (s - us);
+  }
+  f[0] = g0 * g1;
+  f[1] = g0 * g1 * g1 + g2;
+  f[2] = g1 * (e + g2);
+  mine = ((right ? so : s) > 0.0 || us > 0.0) != right;
+}
+
+__device__ inline double pick(const double a[3], int v) { return v == 0 ? a[0] : v == 1 ? a[1] : a[2]; }
+
+template <int N, int R>
+__global__ __launch_bounds__(1024) void dg1d_lds_run_kernel(Geometry G, Tables T, RunArgs A) {
+  extern __shared__ double lds[];
+  const int nx = G.nx, nf = nx + 1, n3 = 3 * N * nx, tid = threadIdx.x, nt = blockDim.x;
+  const Lds s = lds_layout<N>(lds, nx);
+  const double gamma = G.gamma, oneoverdx = G.oneoverdx;
+  const bool source = G.source == 2;
+  const double* k = A.coef;
+  for (int q = tid; q < n3; q += nt) {
+    const int iv = q / nx, c = q - iv * nx;
+    s.st[q] = A.d[(size_t)3 * N * c + iv];
+    s.ue[q] = G.ueq[(size_t)3 * N * c + iv];
+  }
+  for (int q = tid; q < N * nx; q += nt) s.px[q] = A.phx[(size_t)(q % nx) * N * N + q / nx];
+  for (int q = tid; q < 3 * nf; q += nt) s.uf[q] = G.ufe[3 * (q % nf) + q / nf];
+  if (tid < N * N) {
+    s.phq[tid] = T.phq[tid];
+    s.dphq[tid] = T.dphq[tid];
+  }
+  if (tid < 2 * N) s.plr[tid] = T.plr[tid];
+  __syncthreads();
+
+  // this thread's (mode i, variable v, cell c), R of them, and their constants
+  double d[R], w2[R], c1[R], c2[R], c3[R];
+  int mode[R], var[R], cell[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    d[r] = w2[r] = c1[r] = c2[r] = c3[r] = 0.0;
+    const int q = tid + r * nt, iv = q / nx, c = q - iv * nx, i = iv / 3, v = iv - 3 * i;
+    mode[r] = i;
+    var[r] = v;
+    cell[r] = c;
+    __builtin_amdgcn_sched_barrier(0);
+    if (q >= n3) continue;
+    double fve = 0.0, sve = 0.0;
+    for (int j = 0; j < N; ++j) {
+      double e[3], fe[3];
+      for (int w = 0; w < 3; ++w) e[w] = s.ue[(3 * j + w) * nx + c];
+      fv1d::flux(gamma, e, fe);
+      fve = fve + pick(fe, v) * s.dphq[i * N + j] * T.wq[j];
+      if (source) {
+        double se[3];
+        source_term(gamma, e, se);
+        sve = sve + pick(se, v) * s.phq[i * N + j] * T.wq[j] * 0.5;
+      }
+    }
+    const double pl = s.plr[2 * i], pr = s.plr[2 * i + 1];
+    d[r] = s.st[q];
+    c1[r] = oneoverdx * fve;
+    c2[r] = oneoverdx * (G.ffe[3 * (c + 1) + v] * pr - G.ffe[3 * c + v] * pl);
+    c3[r] = sve;
+  }
+
+  double t = A.clk->t, dt = 0.0, dtl = A.clk->dt_last;
+  const int32_t start = A.clk->steps;
+  int32_t steps = start;
+  uint32_t err = A.clk->err;
+  const int faces = (2 * (nx - 1) + 63) / 64 * 64;   // whole waves of lane pairs, so that no wave mixes the two
+  while (err == 0 && steps < A.step_limit && t < A.t_end) {
+#pragma unroll 1
+    for (int stage = 0; stage < 5; ++stage) {
+      double cm = 0.0;
+      const int items = faces + N * nx + (stage == 0 ? nx : 0);
+#pragma unroll 1
+      for (int a = tid; a < items; a += nt) {
+        if (a < faces) {
+          const int f = a / 2 + 1;
+          if (f >= nx) continue;
+          const bool right = a & 1;
+          double u[3], fl[3];
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+            double tr = 0.;
+#pragma unroll
+            for (int i = 0; i < N; ++i) tr = tr + s.st[(3 * i + v) * nx + f - 1 + right] * s.plr[2 * i + 1 - right];
+            u[v] = s.uf[v * nf + f] + tr;
+          }
+          bool mine;
+          pair_flux(gamma, G.riemann, right, u, fl, mine);
+          if (mine) {
+#pragma unroll
+            for (int v = 0; v < 3; ++v) s.F[v * nf + f] = fl[v];
+          }
+        } else if (a < faces + N * nx) {
+          const int b = a - faces, j = b / nx, c = b - j * nx;
+          double us[3], f[3];
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+            double u = 0.0;
+#pragma unroll
+            for (int i = 0; i < N; ++i) u = u + s.st[(3 * i + v) * nx + c] * s.phq[i * N + j];
+            us[v] = s.ue[(3 * j + v) * nx + c] + u;
+          }
+          fv1d::flux(gamma, us, f);
+#pragma unroll
+          for (int v = 0; v < 3; ++v) s.fq[(3 * j + v) * nx + c] = f[v];
+          if (source) {
+            double w[3];
+            source_term(gamma, us, w);
+            s.sq[2 * j * nx + c] = w[1];
+            s.sq[(2 * j + 1) * nx + c] = w[2];
+          }
+        } else {
+          // |v| + c at the first Gauss point of uinit (compute_max_speed :1136-1152)
+          const int c = a - faces - N * nx;
+          double u[3];
+#pragma unroll
+          for (int v = 0; v < 3; ++v) {
+            double w = 0.0;
+#pragma unroll
+            for (int q = 0; q < N; ++q) w = w + s.st[(3 * q + v) * nx + c] * s.px[q * nx + c];
+            u[v] = steps == start ? A.uinit[(size_t)3 * N * c + v] : s.ue[v * nx + c] + w;
+          }
+          cm = fmax(cm, fv1d::speed(gamma, u));
+        }
+      }
+      if (stage == 0) {
+        for (int off = 32; off > 0; off >>= 1) cm = fmax(cm, __shfl_xor(cm, off));
+        if ((tid & 63) == 0) s.red[tid >> 6] = cm;
+      }
+      __syncthreads();
+      if (stage == 0) {
+        double cmax = 0.0;
+        for (int w = 0; w < nt / 64; ++w) cmax = fmax(cmax, s.red[w]);
+        dt = (double)0.9f * A.dx / cmax / (2.0 * (double)N + 1.0);   // :197
+        if (!(dt > 0.0) || !isfinite(dt)) {
+          err = 1;
+          break;
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int q = tid + r * nt, c = cell[r], i = mode[r], v = var[r];
+        __builtin_amdgcn_sched_barrier(0);           // one item's values at a time
+        if (q >= n3) continue;
+        double L = 0.0;                              // dudt(:,:,1) = dudt(:,:,nx) = 0 (:2027-2028)
+        if (c != 0 && c != nx - 1) {
+          double fv = 0.0, sv = 0.0;
+#pragma unroll(R > 1 && N > 3 ? 1 : N)
+          for (int j = 0; j < N; ++j) {
+            fv = fv + s.fq[(3 * j + v) * nx + c] * s.dphq[i * N + j] * T.wq[j];
+            if (source && v > 0) sv = sv + s.sq[(2 * j + v - 1) * nx + c] * s.phq[i * N + j] * T.wq[j] * 0.5;
+          }
+          const double pl = s.plr[2 * i], pr = s.plr[2 * i + 1];
+          L = oneoverdx * fv - c1[r] - oneoverdx * (s.F[v * nf + c + 1] * pr - s.F[v * nf + c] * pl) + c2[r] + sv -
+              c3[r];                                 // :2015-2025
+        }
+        // :264-288, each line as written: (c*dt)*dudt added last
+        const double in = s.st[q];
+        double out;
+        if (stage == 0) {
+          out = d[r] + k[0] * dt * L;
+        } else if (stage == 1) {
+          out = w2[r] = k[1] * d[r] + k[2] * in + k[3] * dt * L;
+        } else if (stage == 2) {
+          out = k[4] * d[r] + k[5] * w2[r] + k[6] * dt * L;
+        } else if (stage == 3) {
+          out = k[7] * d[r] + k[8] * in + k[9] * dt * L;
+          w2[r] = k[10] * w2[r] + k[11] * in + k[12] * dt * L;   // the last line's first terms
+        } else {
+          out = d[r] = w2[r] + k[13] * in + k[14] * dt * L;
+        }
+        s.st[q] = out;
+      }
+      __syncthreads();
+    }
+    if (err) break;
+    t = t + dt;
+    dtl = dt;
+    ++steps;
+  }
+  // the modes, and uinit = u_eq + the modes at legendre(x_quad) (:303-330)
+  if (steps > start)
+    for (int q = tid; q < n3; q += nt) {
+      const int iv = q / nx, c = q - iv * nx, i = iv / 3, v = iv - 3 * i;
+      double a = 0.0;
+      for (int m = 0; m < N; ++m) a = a + s.st[(3 * m + v) * nx + c] * A.phx[((size_t)c * N + i) * N + m];
+      A.d[(size_t)3 * N * c + iv] = s.st[q];
+      A.uinit[(size_t)3 * N * c + iv] = s.ue[q] + a;
+    }
+  if (tid == 0) {
+    A.clk->t = t;
+    A.clk->dt_last = dtl;
+    A.clk->steps = steps;
+    A.clk->err = err;
+  }
+}
+
 }  // namespace dg1d
 
 using namespace dg1d;
@@ -386,6 +651,7 @@ struct fvwb_dg1d {
   Clock* d_clk = nullptr;
   bool loaded = false;
   Tables tab{};
+  size_t lds = 0;             // bytes of LDS a workgroup may have
   double coef[15];
   std::string err;
 };
@@ -445,9 +711,14 @@ extern "C" int fvwb_dg1d_create(fvwb_dg1d_handle* out, const fvwb_dg1d_params* p
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
     return faildg1d(nullptr, FVWB_ERR_HIP, "no HIP device");
+  int dev = 0, lds = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+    return faildg1d(nullptr, FVWB_ERR_HIP, "device query failed");
   fvwb_dg1d* h = new (std::nothrow) fvwb_dg1d;
   if (!h) return faildg1d(nullptr, FVWB_ERR_OOM, "host allocation failed");
   h->p = *p;
+  h->lds = (size_t)lds;
   const int n = p->n, nx = p->nx;
   double chsi[MAXN], w[MAXN];
   gl_quadrature(n, chsi, w);
@@ -571,7 +842,7 @@ extern "C" int fvwb_dg1d_upload(fvwb_dg1d_handle h, const double* delta_u, const
 }
 
 template <int N>
-static void launch_run(fvwb_dg1d* h, int32_t limit, double t_end) {
+static hipError_t launch_run(fvwb_dg1d* h, int32_t limit, double t_end) {
   RunArgs R;
   R.d = run_array(h, 0);
   R.w1 = run_array(h, 1);
@@ -586,7 +857,23 @@ static void launch_run(fvwb_dg1d* h, int32_t limit, double t_end) {
   R.t_end = t_end;
   R.dx = h->p.boxlen / (double)h->p.nx;
   for (int i = 0; i < 15; ++i) R.coef[i] = h->coef[i];
-  hipLaunchKernelGGL(dg1d_run_kernel<N>, dim3(1), dim3(256), 0, h->stream, geometry(h, h->d_ueq), h->tab, R);
+  // the LDS form, the faster one at every size that fits
+  const size_t nx = (size_t)h->p.nx, bytes = sizeof(double) * lds_doubles(N, nx), modes = 3 * N * nx;
+  const size_t points = (2 * (nx - 1) + 63) / 64 * 64 + (N + 1) * nx, most = std::max(points, modes);
+  const unsigned threads = (unsigned)std::min<size_t>(1024, (most + 63) / 64 * 64);
+  if (bytes <= h->lds && modes <= 5 * 1024) {
+    auto* kernel = modes <= threads ? dg1d_lds_run_kernel<N, 1>
+                   : modes <= 2 * 1024 ? dg1d_lds_run_kernel<N, 2>
+                   : modes <= 3 * 1024 ? dg1d_lds_run_kernel<N, 3> : dg1d_lds_run_kernel<N, 5>;
+    if (bytes > 65536) {
+      const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(threads), bytes, h->stream, geometry(h, h->d_ueq), h->tab, R);
+  } else {
+    hipLaunchKernelGGL(dg1d_run_kernel<N>, dim3(1), dim3(256), 0, h->stream, geometry(h, h->d_ueq), h->tab, R);
+  }
+  return hipGetLastError();
 }
 
 // Steps are launched in chunks of at most this many, so one launch stays short.
@@ -603,15 +890,16 @@ extern "C" int fvwb_dg1d_advance(fvwb_dg1d_handle h, int32_t nsteps, double t_en
     if (clk.err) return faildg1d(h, FVWB_ERR_NONPHYSICAL, "wave-speed maximum or dt not finite and positive");
     if (!(clk.t < t_end) || clk.steps >= target) return FVWB_OK;
     const int32_t limit = (int32_t)std::min<int64_t>(target, (int64_t)clk.steps + kChunk);
+    hipError_t launched;
     switch (h->p.n) {
-      case 1: launch_run<1>(h, limit, t_end); break;
-      case 2: launch_run<2>(h, limit, t_end); break;
-      case 3: launch_run<3>(h, limit, t_end); break;
-      case 4: launch_run<4>(h, limit, t_end); break;
-      case 5: launch_run<5>(h, limit, t_end); break;
-      default: launch_run<6>(h, limit, t_end); break;
+      case 1: launched = launch_run<1>(h, limit, t_end); break;
+      case 2: launched = launch_run<2>(h, limit, t_end); break;
+      case 3: launched = launch_run<3>(h, limit, t_end); break;
+      case 4: launched = launch_run<4>(h, limit, t_end); break;
+      case 5: launched = launch_run<5>(h, limit, t_end); break;
+      default: launched = launch_run<6>(h, limit, t_end); break;
     }
-    HIPD(h, hipGetLastError());
+    HIPD(h, launched);
     HIPD(h, hipMemcpyAsync(&clk, h->d_clk, sizeof clk, hipMemcpyDeviceToHost, h->stream));
     HIPD(h, hipStreamSynchronize(h->stream));
   }

@@ -48,4 +48,23 @@ __host__ __device__ inline void llflux(double gamma, const double ul[3], const d
   for (int k = 0; k < 3; ++k) out[k] = 0.5 * (fr[k] + fl[k]) - 0.5 * cmax * (ur[k] - ul[k]);
 }
 
+// the value of the other lane of a pair (even, odd)
+__device__ inline double other(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xb1, 0xf, 0xf, true);   // quad_perm 1,0,3,2
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xb1, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// flux and llflux by a pair of lanes, the even one with the left state and the
+// odd one with the right; both return the numerical flux
+__device__ inline void pair_llflux(double gamma, bool right, const double u[3], double out[3]) {
+  double f[3];
+  flux(gamma, u, f);
+  const double sp = speed(gamma, u), cmax = fmax(sp, other(sp));
+  for (int v = 0; v < 3; ++v) {
+    const double fo = other(f[v]), uo = other(u[v]);
+    out[v] = 0.5 * (fo + f[v]) - 0.5 * cmax * (right ? u[v] - uo : uo - u[v]);
+  }
+}
+
 }  // namespace fv1d

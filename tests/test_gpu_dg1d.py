@@ -131,6 +131,27 @@ def test_run_matches_oracle_bitwise(n, riemann):
     same(u, uo, "u_init")
 
 
+@pytest.mark.parametrize("riemann", [po.DG1D_RIEMANN_LLF, po.DG1D_RIEMANN_HLLC])
+@pytest.mark.parametrize("n,nx", [(1, 3), (3, 4), (2, 33), (3, 113), (3, 114), (3, 227), (3, 228), (6, 60), (5, 250), (3, 341),
+                                  (3, 342), (3, 500), (3, 700)])
+def test_run_sizes_match_oracle_bitwise(n, nx, riemann):
+    """Grids at the edges of one, two, three and five items per thread, of the
+    64 KB that need no attribute, and past what a workgroup's LDS holds."""
+    say(f"case: 1D DG RKi run n={n} nx={nx} riemann={riemann} 6 steps")
+    op = po.make_dg1d_params(nx, n=n, riemann=riemann)
+    d0, e, u0 = po.dg1d_initial(op, ninit=8, pert=1e-2)
+    do, uo, to, ko, ts, dts = po.dg1d_run_rki(op, d0, e, u0, 10.0, max_steps=6)
+    with fvwb.SolverDG1D(gpu_p(op)) as s:
+        s.upload(d0, e, u0)
+        s.advance(2)
+        s.advance(4)
+        t, dtl, k = s.time()
+        d, u = s.download()
+    assert k == ko == 6 and t == to and dtl == dts[-1]
+    same(d, do, "modes")
+    same(u, uo, "u_init")
+
+
 def test_run_in_pieces_equals_one_run():
     say("case: 1D DG RKi run in pieces")
     op = po.make_dg1d_params(64)
