@@ -66,6 +66,7 @@ struct fvwb_ctx {
   int parity = 0;
   bool uploaded = false;
   Tune tune{16, 2};
+  int short_rows = 0;       // strips of 1 or 2 rows instead (small grids; 0: tune.rows)
   std::string err;
 };
 
@@ -179,12 +180,14 @@ extern "C" int fvwb_create(fvwb_handle* out, const fvwb_params* p) {
     fvwb_destroy(h);
     return FVWB_ERR_HIP;
   }
-  // launch shape: rows per wave strip so that a 2048^2 grid yields >= 4k waves
-  long long cells = (long long)nx * ny;
-  // launch shape: short strips keep >= ~16 waves per CU on mid-size grids;
-  // FP32 lanes own 2 columns (8-byte loads leave registers for a deeper ring)
-  h->tune.rows = cells >= (1ll << 24) ? 16 : (cells >= (1ll << 20) ? 8 : 4);
+  // launch shape: short strips keep >= ~16 waves per CU on mid-size grids (FP32,
+  // SSP-RK3: 1200 x 900 54 us per step with four rows and 63 with eight, 2048^2
+  // 127 and 126, FP64 275 and 266); FP32 lanes own 2 columns (8-byte loads leave
+  // registers for a deeper ring)
+  const long long cells = (long long)nx * ny, ntx = (nx + 123) / 124;
+  h->tune.rows = cells >= (1ll << 24) ? 16 : (cells >= (1ll << 22) ? 8 : 4);
   h->tune.cpl = 2;
+  h->short_rows = short_strip_rows(ntx * ny, ntx * ((ny + 1) / 2), false);
   *out = h;
   return FVWB_OK;
 }
@@ -214,7 +217,7 @@ static StageArgs<T> base_args(fvwb_ctx* h) {
   a.rxf = h->rxf; a.rxc = h->rxc; a.eyc = h->eyc; a.eyf = h->eyf;
   a.ctrl = h->ctrl;
   a.plane = h->plane; a.pitch = h->pitch; a.nx = p.nx; a.ny = p.ny;
-  a.rows = h->tune.rows;
+  a.rows = h->short_rows ? h->short_rows : h->tune.rows;
   const int cpl = sizeof(T) == 8 ? 2 : h->tune.cpl;
   const int cols = 62 * cpl;   // columns per wave strip
   a.ntx = (p.nx + cols - 1) / cols;
@@ -539,6 +542,7 @@ extern "C" int fvwb_set_launch(fvwb_handle h, int32_t rows_per_strip, int32_t co
   if (columns_per_lane != 2 && columns_per_lane != 4)
     return fail(h, FVWB_ERR_ARG, "columns_per_lane must be 2 or 4");
   h->tune.rows = rows_per_strip;
+  h->short_rows = 0;
   if (h->p.precision == FVWB_FP32) h->tune.cpl = columns_per_lane;
   return FVWB_OK;
 }

@@ -23,6 +23,11 @@ hipError_t launch_fv2d_batch_f64(const BatchArgs<double>& b, int blocks, int rec
                                  hipStream_t s);
 hipError_t launch_fv2d_batch_f32(const BatchArgs<float>& b, int blocks, int recon, int flux, int bc, int mode,
                                  int cpl, hipStream_t s);
+// strips of one or two rows (fvwb_fv2d_short.hip)
+hipError_t launch_fv2d_batch_short_f64(const BatchArgs<double>& b, int blocks, int recon, int flux, int bc, int mode,
+                                       hipStream_t s);
+hipError_t launch_fv2d_batch_short_f32(const BatchArgs<float>& b, int blocks, int recon, int flux, int bc, int mode,
+                                       hipStream_t s);
 template <typename T>
 hipError_t launch_aos_to_dev(const double* u, const double* w, T* out, int nx, int ny, int pitch, long long plane,
                              double gamma, hipStream_t s);
@@ -67,6 +72,8 @@ struct fvwb_batch {
   int* d_tile_start = nullptr;
   int ntiles = 0;
   int rows = 8, cpl = 2, blocks = 0;    // launch shape (blocks 0 = automatic)
+  bool rows_set = false;                // by the caller: rows as given, else 4 may stand for 1 or 2
+  int strip_rows = 8;                   // rows of the strips as laid out
   int parity = 0;
   bool ready = false;
   bool use_graph = true;
@@ -100,6 +107,13 @@ static void drop_graphs(fvwb_batch* h) {
     if (h->graph[k]) { (void)hipGraphExecDestroy(h->graph[k]); h->graph[k] = nullptr; }
 }
 
+// strips of the whole batch at `rows` rows and two columns per lane
+static long long strips(const fvwb_batch* h, int rows) {
+  long long n = 0;
+  for (const fvwb_params& p : h->p) n += (long long)((p.nx + 123) / 124) * ((p.ny + rows - 1) / rows);
+  return n;
+}
+
 // Strip layout for the current launch shape: per-instance descriptors and the
 // prefix sums of tiles, uploaded to the device.
 static int build_layout(fvwb_batch* h) {
@@ -107,6 +121,9 @@ static int build_layout(fvwb_batch* h) {
   std::vector<int> start(h->ninst);
   long long total = 0;
   const int cpl = h->shared.precision == FVWB_FP64 ? 2 : h->cpl;
+  const bool free_rows = h->rows == 4 && cpl == 2 && !h->rows_set && h->shared.flux == FVWB_FLUX_HLL;
+  const int few = free_rows ? short_strip_rows(strips(h, 1), strips(h, 2), true) : 0;
+  h->strip_rows = few ? few : h->rows;
   for (int b = 0; b < h->ninst; ++b) {
     const fvwb_params& p = h->p[b];
     InstDesc& q = d[b];
@@ -114,9 +131,9 @@ static int build_layout(fvwb_batch* h) {
     q.pitch = row_stride(h, b);
     q.plane = var_stride(h, b);
     q.nx = p.nx; q.ny = p.ny;
-    q.rows = h->rows;
+    q.rows = h->strip_rows;
     q.ntx = (p.nx + 62 * cpl - 1) / (62 * cpl);
-    q.ntiles = q.ntx * ((p.ny + h->rows - 1) / h->rows);
+    q.ntiles = q.ntx * ((p.ny + h->strip_rows - 1) / h->strip_rows);
     q.tx_off = h->txo[b]; q.ty_off = h->tyo[b];
     const double dx = p.boxlen_x / p.nx, dy = p.boxlen_y / p.ny;
     q.h = dx < dy ? dx : dy;
@@ -211,8 +228,14 @@ extern "C" int fvwb_batch_create(fvwb_batch_handle* out, int32_t ninst, const fv
     fvwb_batch_destroy(h);
     return bfail(nullptr, FVWB_ERR_HIP, "table upload failed");
   }
-  // default launch shape: short strips (many waves), FP32 lanes own 2 columns
-  h->rows = 8;
+  // default launch shape: short strips (many waves), FP32 lanes own 2 columns.
+  // Four rows (or fewer, by build_layout) until they make four strips per SIMD:
+  // 2,500 of them ran 30 instances up to 400^2 in 61 us per FP32 step against
+  // 71 with eight rows, 4,350 of them 20 up to 700^2 in 91 against 89
+  // Rusanov batches keep eight: that flux rounds differently (by an ulp) upward
+  // and downward, so its results depend on the strips, and an instance of a batch
+  // equals the problem alone on strips of eight bit for bit
+  h->rows = s0.flux == FVWB_FLUX_HLL && strips(h, 4) <= 4096 ? 4 : 8;
   h->cpl = 2;
   int rc = build_layout(h);
   if (rc) { g_batch_err = h->err; fvwb_batch_destroy(h); return rc; }
@@ -324,10 +347,13 @@ static int enqueue_batch_steps(fvwb_batch* h, int nsteps, double t_end) {
   int blocks = h->blocks > 0 ? h->blocks : (h->ntiles + 3) / 4;
   blocks = std::max(1, std::min(blocks, (h->ntiles + 3) / 4));
   auto launch = [&](const BatchArgs<T>& b, int mode) {
+    const bool few = h->strip_rows <= 2;
     if constexpr (sizeof(T) == 8)
-      return launch_fv2d_batch_f64(b, blocks, s.recon, s.flux, s.bc, mode, h->stream);
+      return few ? launch_fv2d_batch_short_f64(b, blocks, s.recon, s.flux, s.bc, mode, h->stream)
+                 : launch_fv2d_batch_f64(b, blocks, s.recon, s.flux, s.bc, mode, h->stream);
     else
-      return launch_fv2d_batch_f32(b, blocks, s.recon, s.flux, s.bc, mode, h->cpl, h->stream);
+      return few ? launch_fv2d_batch_short_f32(b, blocks, s.recon, s.flux, s.bc, mode, h->stream)
+                 : launch_fv2d_batch_f32(b, blocks, s.recon, s.flux, s.bc, mode, h->cpl, h->stream);
   };
   for (int n = 0; n < nsteps; ++n) {
     a.parity = h->parity;
@@ -459,6 +485,7 @@ extern "C" int fvwb_batch_set_launch(fvwb_batch_handle h, int32_t rows, int32_t 
   h->rows = rows;
   if (h->shared.precision == FVWB_FP32) h->cpl = cpl;
   h->blocks = blocks;
+  h->rows_set = true;
   return build_layout(h);
 }
 
@@ -540,7 +567,7 @@ extern "C" int fvwb_batch_autotune(fvwb_batch_handle h, int32_t trial_steps, con
     int rc = FVWB_OK;
     for (int ci = 0; ci < ncpl && rc == FVWB_OK; ++ci)
       for (int r : row_opts) {
-        h->rows = r; h->cpl = cpl_opts[ci]; h->blocks = 0;
+        h->rows = r; h->cpl = cpl_opts[ci]; h->blocks = 0; h->rows_set = false;
         rc = build_layout(h);
         if (rc) break;
         rc = enqueue_steps(h, 1, INFINITY);  // warm the kernel
@@ -570,7 +597,7 @@ extern "C" int fvwb_batch_autotune(fvwb_batch_handle h, int32_t trial_steps, con
     if (rc) return rc;
     cache_store(cache_path, key, rows, cpl, blocks, best / trial_steps);
   }
-  h->rows = rows; h->cpl = cpl; h->blocks = blocks;
+  h->rows = rows; h->cpl = cpl; h->blocks = blocks; h->rows_set = false;
   int rc = build_layout(h);
   if (rc) return rc;
   if (rows_out) *rows_out = rows;

@@ -69,6 +69,19 @@ struct BatchArgs {
   double t_end, alpha, beta;
 };
 
+// Strips of one or two rows (0: neither), given how many strips of each there
+// would be.  While every strip has a SIMD of its own a stage lasts as long as
+// one strip, and one row is the shortest: SSP-RK3 in FP64 at 300^2 takes 24 us
+// per step with one row, 28 with two, 41 with four.  With more strips the rows
+// read twice begin to count: at 500 x 250 30, 28 and 40 us, at 1000^2 (4,500
+// strips of two rows) 104, 87 and 92, at 1500^2 (9,750) 205, 161 and 152.  A
+// batch looks its instance up per strip: 16 instances up to 300^2 (1,370 strips
+// of two rows) take 34 us with two rows and 37 with four in FP32, 30 up to
+// 400^2 (5,000) 69 and 61.
+inline int short_strip_rows(long long one, long long two, bool batch) {
+  return one <= 1024 ? 1 : two <= (batch ? 3072 : 5120) ? 2 : 0;
+}
+
 // Launch configuration chosen by the tuner.
 struct Tune {
   int rows;  // rows per wave strip

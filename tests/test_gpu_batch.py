@@ -57,6 +57,27 @@ def test_batch_equals_single_instances_bitwise(prec, scheme):
             assert np.array_equal(bt.download_deviation(k), dev_s), k
 
 
+@pytest.mark.parametrize("prec", (fvwb.FP64, fvwb.FP32))
+def test_batch_of_short_strips_equals_single_instances_bitwise(prec):
+    """A batch whose strips have two rows, set to four and back by the tuner."""
+    sizes = [(300, 301), (248, 250), (40, 333), (310, 270)]
+    say(f"case: batch of two-row strips prec={prec}")
+    ps = inst_params(prec, sizes=sizes, gs=GS[:4])
+    amps = np.array([1e-3, 1e-2, 5e-3, 1e-4])
+    with fvwb.Batch2D(ps) as bt, fvwb.Batch2D(ps) as b4:
+        b4.set_launch(4, 2)
+        for b in (bt, b4):
+            b.init_gaussian(amps)
+            b.advance(5)
+        assert bt.get_launch()[:2] == b4.get_launch()[:2] == (4, 2)
+        assert bt.get_launch()[3] > b4.get_launch()[3]
+        for k, p in enumerate(ps):
+            dev_s, (ts, dts, ns) = single_run(p, amps[k], 5)
+            for b in (bt, b4):
+                assert b.time(k) == (ts, dts, ns)
+                np.testing.assert_array_equal(b.download_deviation(k), dev_s)
+
+
 def test_batch_fp64_matches_oracle():
     say("case: batch FP64 instances vs oracle")
     ps = inst_params(fvwb.FP64, sizes=SIZES[:4], gs=GS[:4])

@@ -358,3 +358,34 @@ def test_advance_past_t_end_then_further(precision):
         b.advance(2000, 0.025)
         assert a.time() == b.time()
         assert np.array_equal(a.download_deviation(), b.download_deviation())
+
+
+@pytest.mark.parametrize("precision", [fvwb.FP64, fvwb.FP32])
+@pytest.mark.parametrize("shape", [(4, 4), (125, 512), (125, 513), (130, 77), (700, 301), (1000, 1000)])
+def test_short_strips_equal_long_ones(shape, precision):
+    """The one- and two-row strips that small grids get (1024 strips of one row
+    and one more, odd heights, the two-row range) against strips of eight: bit
+    for bit with HLL.  Rusanov rounds by an ulp of the deviation per stage
+    differently upward and downward, so there the bound is one per stage."""
+    nx, ny = shape
+    for flux in (fvwb.FLUX_HLL, fvwb.FLUX_RUSANOV):
+        for recon, bc, integ, stages in ((fvwb.RECON_MUSCL_MINMOD, fvwb.BC_REFLECT, fvwb.SSPRK3, 3),
+                                         (fvwb.RECON_FIRST_ORDER, fvwb.BC_FROZEN_RING, fvwb.RK2_HEUN, 2)):
+            say(f"case: short strips {nx}x{ny} precision={precision} flux={flux} recon={recon} bc={bc}")
+            p = fvwb.make_params(nx, ny, recon=recon, flux=flux, bc=bc, integrator=integ, precision=precision, rho0=1.0,
+                                 g=1.3)
+            out = []
+            for rows in (0, 8):
+                with fvwb.Solver2D(p) as s:
+                    if rows:
+                        s.set_launch(rows, 2)
+                    s.init_gaussian(1e-2, 0.4, 0.6, 80.0)
+                    s.advance(6)
+                    out.append((s.download_deviation(), s.time()))
+            (a, ta), (b, tb) = out
+            if flux == fvwb.FLUX_HLL:
+                np.testing.assert_array_equal(a, b)
+                assert ta == tb
+            else:
+                eps = np.finfo(np.float64 if precision == fvwb.FP64 else np.float32).eps
+                np.testing.assert_allclose(a, b, rtol=0, atol=6 * stages * eps * np.max(np.abs(b)))
