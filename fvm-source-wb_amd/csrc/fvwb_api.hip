@@ -14,6 +14,7 @@
 #include "../../include/fvwb.h"
 #include "fvwb_checkpoint.h"
 #include "fvwb_internal.h"
+#include "fvwb_transfer.h"
 
 namespace fvwb {
 hipError_t launch_fv2d_stage_f64(const StageArgs<double>& a, int recon, int flux, int bc, int mode, hipStream_t s);
@@ -65,6 +66,7 @@ struct fvwb_ctx {
   unsigned long long* red = nullptr;
   int parity = 0;
   bool uploaded = false;
+  fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   Tune tune{16, 2};
   int short_rows = 0;       // strips of 1 or 2 rows instead (small grids; 0: tune.rows)
   std::string err;
@@ -248,8 +250,8 @@ static int residual_host(fvwb_handle h, const double* u, const double* w_eq, dou
   if (rc) return rc;
   const fvwb_params& p = h->p;
   const size_t bytes = 4 * (size_t)p.nx * p.ny * sizeof(double);
-  FVWB_HIP(h, hipMemcpyAsync(h->stage_u, u, bytes, hipMemcpyHostToDevice, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(h->stage_w, w_eq, bytes, hipMemcpyHostToDevice, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage_u, u, bytes, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage_w, w_eq, bytes, h->stream));
   FVWB_HIP(h, launch_aos_to_dev<double>(h->stage_u, h->stage_w, h->res_in, p.nx, p.ny, h->pitch, h->plane, p.gamma,
                                         h->stream));
   StageArgs<double> a = base_args<double>(h);
@@ -258,7 +260,7 @@ static int residual_host(fvwb_handle h, const double* u, const double* w_eq, dou
   FVWB_HIP(h, launch_fv2d_stage_f64(a, p.recon, p.flux, p.bc, 0, h->stream));
   FVWB_HIP(h, launch_dev_to_aos<double>(h->res_out, nullptr, h->stage_u, p.nx, p.ny, h->pitch, h->plane, p.gamma,
                                         false, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(dudt, h->stage_u, bytes, hipMemcpyDeviceToHost, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_host(h->xfer, dudt, h->stage_u, bytes, h->stream));
   FVWB_HIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -280,9 +282,9 @@ extern "C" int fvwb_compute_update(fvwb_handle h, const double* u, const double*
   if (rc) return rc;
   const fvwb_params& p = h->p;
   const size_t bytes = 4 * (size_t)p.nx * p.ny * sizeof(double);
-  FVWB_HIP(h, hipMemcpyAsync(h->stage_u, u, bytes, hipMemcpyHostToDevice, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage_u, u, bytes, h->stream));
   FVWB_HIP(h, launch_plain_update(h->stage_u, h->stage_w, p.nx, p.ny, p.gamma, p.boxlen_x, p.boxlen_y, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(dudt, h->stage_w, bytes, hipMemcpyDeviceToHost, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_host(h->xfer, dudt, h->stage_w, bytes, h->stream));
   FVWB_HIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -291,7 +293,7 @@ extern "C" int fvwb_compute_max_speed(fvwb_handle h, const double* u, double* cm
   if (!h || !u || !cmax) return fail(h, FVWB_ERR_ARG, "NULL argument");
   const fvwb_params& p = h->p;
   const size_t n = (size_t)p.nx * p.ny;
-  FVWB_HIP(h, hipMemcpyAsync(h->stage_u, u, 4 * n * sizeof(double), hipMemcpyHostToDevice, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage_u, u, 4 * n * sizeof(double), h->stream));
   FVWB_HIP(h, hipMemsetAsync(h->red, 0, sizeof(unsigned long long), h->stream));
   FVWB_HIP(h, launch_max_speed_aos(h->stage_u, (long long)n, p.gamma, h->red, h->stream));
   unsigned long long bits = 0;
@@ -321,8 +323,8 @@ extern "C" int fvwb_upload(fvwb_handle h, const double* u, const double* w_eq) {
   if (!h || !u || !w_eq) return fail(h, FVWB_ERR_ARG, "NULL argument");
   const fvwb_params& p = h->p;
   const size_t bytes = 4 * (size_t)p.nx * p.ny * sizeof(double);
-  FVWB_HIP(h, hipMemcpyAsync(h->stage_u, u, bytes, hipMemcpyHostToDevice, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(h->w_eq, w_eq, bytes, hipMemcpyHostToDevice, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage_u, u, bytes, h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_device(h->xfer, h->w_eq, w_eq, bytes, h->stream));
   if (p.precision == FVWB_FP64)
     FVWB_HIP(h, launch_aos_to_dev<double>(h->stage_u, h->w_eq, (double*)h->buf[0], p.nx, p.ny, h->pitch, h->plane,
                                           p.gamma, h->stream));
@@ -442,8 +444,7 @@ extern "C" int fvwb_download(fvwb_handle h, double* u) {
   else
     FVWB_HIP(h, launch_dev_to_aos<float>((const float*)h->buf[0], h->w_eq, h->stage_u, p.nx, p.ny, h->pitch,
                                          h->plane, p.gamma, true, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(u, h->stage_u, 4 * (size_t)p.nx * p.ny * sizeof(double), hipMemcpyDeviceToHost,
-                             h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_host(h->xfer, u, h->stage_u, 4 * (size_t)p.nx * p.ny * sizeof(double), h->stream));
   FVWB_HIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -458,8 +459,7 @@ extern "C" int fvwb_download_deviation(fvwb_handle h, double* du) {
   else
     FVWB_HIP(h, launch_dev_to_aos<float>((const float*)h->buf[0], nullptr, h->stage_u, p.nx, p.ny, h->pitch,
                                          h->plane, p.gamma, false, h->stream));
-  FVWB_HIP(h, hipMemcpyAsync(du, h->stage_u, 4 * (size_t)p.nx * p.ny * sizeof(double), hipMemcpyDeviceToHost,
-                             h->stream));
+  FVWB_HIP(h, fvwb_xfer::to_host(h->xfer, du, h->stage_u, 4 * (size_t)p.nx * p.ny * sizeof(double), h->stream));
   FVWB_HIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }

@@ -17,6 +17,7 @@
 
 #include "../../include/fvwb.h"
 #include "fvwb_internal.h"
+#include "fvwb_transfer.h"
 
 namespace fvwb {
 hipError_t launch_fv2d_batch_f64(const BatchArgs<double>& b, int blocks, int recon, int flux, int bc, int mode,
@@ -76,6 +77,7 @@ struct fvwb_batch {
   int strip_rows = 8;                   // rows of the strips as laid out
   int parity = 0;
   bool ready = false;
+  fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   bool use_graph = true;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   double graph_tend[2] = {0.0, 0.0};
@@ -317,8 +319,8 @@ extern "C" int fvwb_batch_upload(fvwb_batch_handle h, int32_t inst, const double
   if (!u || !w_eq) return bfail(h, FVWB_ERR_ARG, "NULL argument");
   const fvwb_params& p = h->p[inst];
   const size_t bytes = 4 * (size_t)p.nx * p.ny * sizeof(double);
-  BATCH_HIP(h, hipMemcpyAsync(h->stage, u, bytes, hipMemcpyHostToDevice, h->stream));
-  BATCH_HIP(h, hipMemcpyAsync(h->w_eq + h->woff[inst], w_eq, bytes, hipMemcpyHostToDevice, h->stream));
+  BATCH_HIP(h, fvwb_xfer::to_device(h->xfer, h->stage, u, bytes, h->stream));
+  BATCH_HIP(h, fvwb_xfer::to_device(h->xfer, h->w_eq + h->woff[inst], w_eq, bytes, h->stream));
   if (h->esize == 8)
     BATCH_HIP(h, launch_aos_to_dev<double>(h->stage, h->w_eq + h->woff[inst], (double*)h->pool[0] + h->off[inst],
                                            p.nx, p.ny, row_stride(h, inst), var_stride(h, inst), p.gamma, h->stream));
@@ -450,8 +452,7 @@ static int download_impl(fvwb_batch* h, int inst, double* u, bool add_eq) {
     BATCH_HIP(h, launch_dev_to_aos<float>((const float*)h->pool[0] + h->off[inst], h->w_eq + h->woff[inst],
                                           h->stage, p.nx, p.ny, row_stride(h, inst), var_stride(h, inst), p.gamma, add_eq,
                                           h->stream));
-  BATCH_HIP(h, hipMemcpyAsync(u, h->stage, 4 * (size_t)p.nx * p.ny * sizeof(double), hipMemcpyDeviceToHost,
-                              h->stream));
+  BATCH_HIP(h, fvwb_xfer::to_host(h->xfer, u, h->stage, 4 * (size_t)p.nx * p.ny * sizeof(double), h->stream));
   BATCH_HIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }

@@ -40,6 +40,7 @@
 #include "../../include/fvwb.h"
 #include "fvwb_checkpoint.h"
 #include "fvwb_device.h"
+#include "fvwb_transfer.h"
 
 namespace fvwb {
 namespace dg {
@@ -858,6 +859,7 @@ static const int MI[6] = {0, 1, 0, 2, 1, 0}, MJ[6] = {0, 0, 1, 0, 1, 2};
 
 struct fvwb_dg {
   fvwb_dg_params p{};
+  fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   hipStream_t stream = nullptr;
   int pitch = 0;
   long long plane = 0;
@@ -1146,7 +1148,7 @@ static void launch_limit(fvwb_dg* h, const LimArgs& a) {
 static int put_modes(fvwb_dg* h, const double* modes, float* dst) {
   const fvwb_dg_params& p = h->p;
   const long long n = 4LL * NM * p.nx * p.ny;
-  DGHIP(h, hipMemcpyAsync(h->host_stage, modes, sizeof(double) * n, hipMemcpyHostToDevice, h->stream));
+  DGHIP(h, fvwb_xfer::to_device(h->xfer, h->host_stage, modes, sizeof(double) * n, h->stream));
   hipLaunchKernelGGL(dg_to_planes_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->host_stage, dst,
                      p.nx, p.ny, h->pitch, h->plane);
   DGHIP(h, hipGetLastError());
@@ -1213,7 +1215,7 @@ extern "C" int fvwb_dg_compute_residual(fvwb_dg_handle h, const double* modes, d
   hipLaunchKernelGGL(dg_from_planes_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->cell(2),
                      h->host_stage, p.nx, p.ny, h->pitch, h->plane);
   DGHIP(h, hipGetLastError());
-  DGHIP(h, hipMemcpyAsync(dudt, h->host_stage, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
+  DGHIP(h, fvwb_xfer::to_host(h->xfer, dudt, h->host_stage, sizeof(double) * n, h->stream));
   DGHIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -1349,7 +1351,7 @@ extern "C" int fvwb_dg_download(fvwb_dg_handle h, double* modes) {
   hipLaunchKernelGGL(dg_from_planes_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->cell(0),
                      h->host_stage, p.nx, p.ny, h->pitch, h->plane);
   DGHIP(h, hipGetLastError());
-  DGHIP(h, hipMemcpyAsync(modes, h->host_stage, sizeof(double) * n, hipMemcpyDeviceToHost, h->stream));
+  DGHIP(h, fvwb_xfer::to_host(h->xfer, modes, h->host_stage, sizeof(double) * n, h->stream));
   DGHIP(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }

@@ -25,6 +25,7 @@
 #include <string>
 
 #include "../../include/fvwb.h"
+#include "fvwb_transfer.h"
 
 #pragma clang fp contract(off)
 
@@ -1193,6 +1194,7 @@ struct fvwb_dgq {
   double* part = nullptr;                    // error partials
   Clock* clk = nullptr;
   bool loaded = false;
+  fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   std::string err;
 };
 
@@ -1396,12 +1398,12 @@ extern "C" int fvwb_dgq_compute_update(fvwb_dgq_handle h, const double* delta_u,
                                        const double* u_eq, double* dudt) {
   (void)u_eq;      // unused by the reference (:1141)
   if (!h || !delta_u || !x || !y || !dudt) return failq(h, FVWB_ERR_ARG, "NULL argument");
-  HIPQ(h, hipMemcpyAsync(h->s_in, delta_u, state_bytes(h), hipMemcpyHostToDevice, h->stream));
-  HIPQ(h, hipMemcpyAsync(h->xi, x, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
-  HIPQ(h, hipMemcpyAsync(h->yi, y, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_in, delta_u, state_bytes(h), h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->xi, x, coord_bytes(h), h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->yi, y, coord_bytes(h), h->stream));
   int rc = gradients(h, h->xi, h->yi, h->gxi, h->gyi);
   if (rc || (rc = stage(h, h->s_in, Coords{h->xi, h->yi, h->gxi, h->gyi}, Epi{}, h->s_out, nullptr))) return rc;
-  HIPQ(h, hipMemcpyAsync(dudt, h->s_out, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
+  HIPQ(h, fvwb_xfer::to_host(h->xfer, dudt, h->s_out, state_bytes(h), h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -1409,7 +1411,7 @@ extern "C" int fvwb_dgq_compute_update(fvwb_dgq_handle h, const double* delta_u,
 extern "C" int fvwb_dgq_compute_max_speed(fvwb_dgq_handle h, const double* u, double* cs_max, double* v_xmax,
                                           double* v_ymax, double* speed_max) {
   if (!h || !u || !cs_max || !v_xmax || !v_ymax || !speed_max) return failq(h, FVWB_ERR_ARG, "NULL argument");
-  HIPQ(h, hipMemcpyAsync(h->s_in, u, sizeof(double) * 4 * (size_t)h->nc, hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_in, u, sizeof(double) * 4 * (size_t)h->nc, h->stream));
   launch_speed(h, h->s_in, h->res, nullptr, 0.0);
   HIPQ(h, hipGetLastError());
   double r[4];
@@ -1424,20 +1426,20 @@ extern "C" int fvwb_dgq_compute_max_speed(fvwb_dgq_handle h, const double* u, do
 
 extern "C" int fvwb_dgq_apply_limiter(fvwb_dgq_handle h, double* u) {
   if (!h || !u) return failq(h, FVWB_ERR_ARG, "NULL argument");
-  HIPQ(h, hipMemcpyAsync(h->s_in, u, state_bytes(h), hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_in, u, state_bytes(h), h->stream));
   int rc = limit(h, h->s_in);
   if (rc) return rc;
-  HIPQ(h, hipMemcpyAsync(u, h->s_in, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
+  HIPQ(h, fvwb_xfer::to_host(h->xfer, u, h->s_in, state_bytes(h), h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
 
 static int project_host(fvwb_dgq* h, const double* src, double* dst, bool to_nodes) {
   if (!h || !src || !dst) return failq(h, FVWB_ERR_ARG, "NULL argument");
-  HIPQ(h, hipMemcpyAsync(h->s_in, src, state_bytes(h), hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_in, src, state_bytes(h), h->stream));
   int rc = project(h, h->s_in, h->s_out, to_nodes);
   if (rc) return rc;
-  HIPQ(h, hipMemcpyAsync(dst, h->s_out, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
+  HIPQ(h, fvwb_xfer::to_host(h->xfer, dst, h->s_out, state_bytes(h), h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -1453,9 +1455,9 @@ extern "C" int fvwb_dgq_nodes_from_modes(fvwb_dgq_handle h, const double* modes,
 extern "C" int fvwb_dgq_upload(fvwb_dgq_handle h, const double* delta_u, const double* x, const double* y) {
   if (!h || !delta_u || !x || !y) return failq(h, FVWB_ERR_ARG, "NULL argument");
   const Clock zero{};
-  HIPQ(h, hipMemcpyAsync(h->du, delta_u, state_bytes(h), hipMemcpyHostToDevice, h->stream));
-  HIPQ(h, hipMemcpyAsync(h->x, x, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
-  HIPQ(h, hipMemcpyAsync(h->y, y, coord_bytes(h), hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->du, delta_u, state_bytes(h), h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->x, x, coord_bytes(h), h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->y, y, coord_bytes(h), h->stream));
   HIPQ(h, hipMemcpyAsync(h->clk, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
   int rc = gradients(h, h->x, h->y, h->gx, h->gy);
   if (rc) return rc;
@@ -1556,7 +1558,7 @@ extern "C" int fvwb_dgq_advance(fvwb_dgq_handle h, int32_t nsteps, double t_end)
 extern "C" int fvwb_dgq_download(fvwb_dgq_handle h, double* delta_u) {
   if (!h || !delta_u) return failq(h, FVWB_ERR_ARG, "NULL argument");
   if (!h->loaded) return failq(h, FVWB_ERR_STATE, "download before upload");
-  HIPQ(h, hipMemcpyAsync(delta_u, h->du, state_bytes(h), hipMemcpyDeviceToHost, h->stream));
+  HIPQ(h, fvwb_xfer::to_host(h->xfer, delta_u, h->du, state_bytes(h), h->stream));
   HIPQ(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -1579,12 +1581,12 @@ extern "C" int fvwb_dgq_compute_error(fvwb_dgq_handle h, const double* nodes, co
   if (!h || !u_init || !linf || !l1 || !l2) return failq(h, FVWB_ERR_ARG, "NULL argument");
   if (!nodes && !h->loaded) return failq(h, FVWB_ERR_STATE, "no nodal values and no uploaded state");
   if (nodes) {
-    HIPQ(h, hipMemcpyAsync(h->s_out, nodes, state_bytes(h), hipMemcpyHostToDevice, h->stream));
+    HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_out, nodes, state_bytes(h), h->stream));
   } else {
     int rc = project(h, h->du, h->s_out, true);
     if (rc) return rc;
   }
-  HIPQ(h, hipMemcpyAsync(h->s_in, u_init, state_bytes(h), hipMemcpyHostToDevice, h->stream));
+  HIPQ(h, fvwb_xfer::to_device(h->xfer, h->s_in, u_init, state_bytes(h), h->stream));
   const long long nb = err_blocks(h->nc);
   if (h->p.order == 2)
     hipLaunchKernelGGL(dgq_error_kernel<2>, dim3((unsigned)nb), dim3(ERR_THREADS), 0, h->stream, h->g, h->T,

@@ -20,6 +20,7 @@
 #include "../../include/fvwb.h"
 #include "fvwb_checkpoint.h"
 #include "fvwb_device.h"
+#include "fvwb_transfer.h"
 
 #pragma clang fp contract(off)
 
@@ -378,6 +379,7 @@ using namespace rd;
 struct fvwb_rd {
   fvwb_rd_params p{};
   Geo g{};
+  fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   hipStream_t stream = nullptr;
   double* buf[2] = {nullptr, nullptr};   // state, AoS(4,nx,ny): buf[par], the other one is the next step's
   int par = 0;                           // parity of the clock's step count
@@ -493,12 +495,12 @@ extern "C" int fvwb_rd_compute_update(fvwb_rd_handle h, const double* u, const d
   if (!h || !u || !diff || !dudt) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
   // the update works in the step's scratch arrays; an uploaded state stays as it is
-  HIPR(h, hipMemcpyAsync(h->d_up, u, nb, hipMemcpyHostToDevice, h->stream));
+  HIPR(h, fvwb_xfer::to_device(h->xfer, h->d_up, u, nb, h->stream));
   double* d_diff = h->buf[h->par ^ 1];
-  HIPR(h, hipMemcpyAsync(d_diff, diff, nb, hipMemcpyHostToDevice, h->stream));
+  HIPR(h, fvwb_xfer::to_device(h->xfer, d_diff, diff, nb, h->stream));
   int rc = sweep<UPDATE>(h, h->d_up, nullptr, nullptr, d_diff, dt, nullptr, h->d_dudt, nullptr);
   if (rc) return rc;
-  HIPR(h, hipMemcpyAsync(dudt, h->d_dudt, nb, hipMemcpyDeviceToHost, h->stream));
+  HIPR(h, fvwb_xfer::to_host(h->xfer, dudt, h->d_dudt, nb, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }
@@ -506,7 +508,7 @@ extern "C" int fvwb_rd_compute_update(fvwb_rd_handle h, const double* u, const d
 extern "C" int fvwb_rd_compute_max_speed(fvwb_rd_handle h, const double* u, double* cmax) {
   if (!h || !u || !cmax) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
-  HIPR(h, hipMemcpyAsync(h->d_up, u, nb, hipMemcpyHostToDevice, h->stream));
+  HIPR(h, fvwb_xfer::to_device(h->xfer, h->d_up, u, nb, h->stream));
   return max_speed(h, h->d_up, cmax);
 }
 
@@ -515,7 +517,7 @@ extern "C" int fvwb_rd_upload(fvwb_rd_handle h, const double* u) {
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
   const Clock zero{};
   h->par = 0;
-  HIPR(h, hipMemcpyAsync(h->buf[0], u, nb, hipMemcpyHostToDevice, h->stream));
+  HIPR(h, fvwb_xfer::to_device(h->xfer, h->buf[0], u, nb, h->stream));
   HIPR(h, hipMemcpyAsync(h->d_clk, &zero, sizeof zero, hipMemcpyHostToDevice, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
   h->loaded = true;
@@ -569,7 +571,7 @@ extern "C" int fvwb_rd_download(fvwb_rd_handle h, double* u) {
   if (!h || !u) return failrd(h, FVWB_ERR_ARG, "NULL argument");
   if (!h->loaded) return failrd(h, FVWB_ERR_STATE, "download before upload");
   const size_t nb = sizeof(double) * 4 * (size_t)h->p.nx * (size_t)h->p.ny;
-  HIPR(h, hipMemcpyAsync(u, h->buf[h->par], nb, hipMemcpyDeviceToHost, h->stream));
+  HIPR(h, fvwb_xfer::to_host(h->xfer, u, h->buf[h->par], nb, h->stream));
   HIPR(h, hipStreamSynchronize(h->stream));
   return FVWB_OK;
 }

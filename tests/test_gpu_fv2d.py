@@ -8,6 +8,7 @@ separable equilibrium tables (e^{-kx} e^{-ky} instead of e^{-k(x+y)}) and the
 deviation storage, all at the level of a few ulp of the O(1) face fluxes
 divided by dx: |d dudt| <= 64*eps*2/dx.  FP32: L1 density error <= 1e-6 (the
 BASELINE accuracy target) and max error <= 1e-6."""
+import ctypes
 import itertools
 import math
 import os
@@ -389,3 +390,35 @@ def test_short_strips_equal_long_ones(shape, precision):
             else:
                 eps = np.finfo(np.float64 if precision == fvwb.FP64 else np.float32).eps
                 np.testing.assert_allclose(a, b, rtol=0, atol=6 * stages * eps * np.max(np.abs(b)))
+
+
+@pytest.mark.parametrize("nx,ny", [(511, 512), (512, 512), (512, 513), (1024, 1023), (1024, 1025), (1303, 1501)])
+def test_large_host_copies_are_exact(nx, ny):
+    """States just below, at and above the sizes from which host threads move
+    them (8 MB to the host, 32 MB to the device), and of an odd byte count per
+    chunk: what went up comes back, from a fresh and from a reused handle, and
+    from an array that the runtime knows."""
+    say(f"case: large host copies {nx}x{ny}")
+    rng = np.random.default_rng(nx + ny)
+    p = fvwb.make_params(nx, ny, rho0=1.0)
+    u = np.asfortranarray(rng.random((4, nx, ny)) + 1.0)
+    w = np.zeros((4, nx, ny), order="F")
+    w[0] = 0.5
+    w[3] = 0.25
+    ueq = np.zeros((4, 1, 1))
+    ueq[0], ueq[3] = 0.5, 0.25 / (p.gamma - 1.0)
+    hip = ctypes.CDLL("libamdhip64.so")
+    pinned = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(pinned), ctypes.c_size_t(u.nbytes), 0) == 0
+    known = np.ctypeslib.as_array(ctypes.cast(pinned, ctypes.POINTER(ctypes.c_double)), (u.size,))
+    known = known.reshape((4, nx, ny), order="F")
+    with fvwb.Solver2D(p) as s:
+        for k in range(3):
+            src = u * (k + 1)
+            if k == 2:
+                known[...] = src
+                src = known
+            s.upload(src, w)
+            np.testing.assert_array_equal(s.download_deviation(), src - ueq)
+    del known, src
+    assert hip.hipHostFree(pinned) == 0
