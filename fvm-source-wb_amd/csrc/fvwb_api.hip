@@ -182,14 +182,24 @@ extern "C" int fvwb_create(fvwb_handle* out, const fvwb_params* p) {
     fvwb_destroy(h);
     return FVWB_ERR_HIP;
   }
-  // launch shape: short strips keep >= ~16 waves per CU on mid-size grids (FP32,
-  // SSP-RK3: 1200 x 900 54 us per step with four rows and 63 with eight, 2048^2
-  // 127 and 126, FP64 275 and 266); FP32 lanes own 2 columns (8-byte loads leave
-  // registers for a deeper ring)
+  // launch shape: short strips keep >= ~16 waves per CU on mid-size grids; FP32
+  // lanes own 2 columns (8-byte loads leave registers for a deeper ring).
+  // Between 2^20 and 2^22 cells a stage lasts as long as the SIMD with most
+  // strips, each about its rows and 2.5 more: with four rows against eight FP32
+  // steps took 54 and 63 us at 1200 x 900, 57 and 65 at 1500 x 900, but 70 and 68
+  // at 1300^2, 96 and 92 at 1700^2.  The FP64 MUSCL kernels, two waves per SIMD,
+  // were within 6 % either way and keep eight.
   const long long cells = (long long)nx * ny, ntx = (nx + 123) / 124;
-  h->tune.rows = cells >= (1ll << 24) ? 16 : (cells >= (1ll << 22) ? 8 : 4);
+  auto strips = [&](int rows) { return ntx * ((ny + rows - 1) / rows); };
+  auto length = [&](int rows) { return (strips(rows) + 1023) / 1024 * (2 * rows + 5); };
+  const bool fp64 = p->precision == FVWB_FP64, muscl = p->recon == FVWB_RECON_MUSCL_MINMOD;
+  h->tune.rows = cells >= (1ll << 24) ? 16 : cells >= (1ll << 22) ? 8 : cells < (1ll << 20) ? 4
+                 : !(fp64 && muscl) && length(4) < length(8) ? 4 : 8;
   h->tune.cpl = 2;
-  h->short_rows = short_strip_rows(ntx * ny, ntx * ((ny + 1) / 2), false);
+  h->short_rows = short_strip_rows(strips(1), strips(2), false);
+  // FP64 strips of four that all run at once, two per SIMD, beat more than three
+  // of two rows: 69 against 73 us at 1000 x 800
+  if (fp64 && h->short_rows == 2 && strips(2) > 3072 && strips(4) <= 2048) h->short_rows = 0;
   *out = h;
   return FVWB_OK;
 }
