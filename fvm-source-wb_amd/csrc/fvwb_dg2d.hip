@@ -1031,7 +1031,12 @@ extern "C" int fvwb_dg_create(fvwb_dg_handle* out, const fvwb_dg_params* p) {
       }
     }
   }
-  // segments along y: as many waves as the device holds at once, at least 4 rows each
+  // segments along y: as many waves as the device holds at once, at least 4 rows
+  // each, or fewer rows while every wave still has a SIMD of its own: a small
+  // grid's stage lasts as long as one wave (24 x 30 43 us per step with four rows
+  // and 30 with one, 100^2 44 and 31); with more waves than SIMDs the rows below
+  // and above a segment cost what they save (300 x 310, SSP(5,4): 119 us with
+  // four rows, 127 with three)
   {
     int dev = 0, cus = 0, blocks_per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -1042,6 +1047,8 @@ extern "C" int fvwb_dg_create(fvwb_dg_handle* out, const fvwb_dg_params* p) {
     const long long slots = 4LL * std::max(1, cus) * std::max(1, blocks_per_cu);
     const long long nseg = std::max(1LL, std::min<long long>(ny, slots / h->ntx));
     h->seg_rows = std::max(4, (int)((ny + nseg - 1) / nseg));
+    for (int r = 3; r >= 1; --r)
+      if ((long long)h->ntx * ((ny + r - 1) / r) <= 4LL * cus) h->seg_rows = r;
     h->nseg = (ny + h->seg_rows - 1) / h->seg_rows;
   }
   if (hipMemcpy(h->exn, ex.data(), sizeof(double) * ex.size(), hipMemcpyHostToDevice) != hipSuccess ||

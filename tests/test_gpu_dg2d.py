@@ -49,6 +49,14 @@ def test_residual_matches_oracle(shape, flux):
     assert err <= 2e-5 * np.max(np.abs(ref))
 
 
+@pytest.mark.parametrize("shape", [(20, 512), (20, 513), (20, 601), (20, 1025), (20, 1300), (20, 2100), (15, 2)])
+def test_residual_matches_oracle_short_segments(shape):
+    """Narrow grids either side of one, two and three rows per segment on a
+    256-CU device (1024 waves), with odd last segments; the bounds are those of
+    the larger grids below."""
+    test_residual_matches_oracle_large(shape)
+
+
 @pytest.mark.parametrize("shape", [(1000, 1030), (2000, 301)])
 def test_residual_matches_oracle_large(shape):
     """Grids large enough that the sweep runs segments of many rows (25 and 15
