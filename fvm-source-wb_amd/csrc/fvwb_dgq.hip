@@ -578,8 +578,8 @@ __global__ __launch_bounds__(256) void dgq_grad_kernel(int gcase, long long n, c
 //      stage w5.
 // Every sum takes its terms in the reference's order.
 //
-// Bound by FP64 issue: about 2,800 vector instructions per wave, 63 % of the
-// issue slots at 512^2 and O = 3, 2.2 TB/s.  One launch instead of the four
+// Bound by FP64 issue: about 2,800 vector instructions per wave, 61 % of the
+// issue slots at 512^2 and O = 3, 2.9 TB/s.  One launch instead of the four
 // (traces, faces, cells, limiter) that moved 400 MB of traces and face fluxes
 // and the state three more times per stage: 125 against 390 us per stage at
 // 512^2, 8 against 32 at 16^2.  Tiles of 16 x 8 cells share more halo but hold
