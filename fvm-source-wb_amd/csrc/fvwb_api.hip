@@ -68,7 +68,7 @@ struct fvwb_ctx {
   bool uploaded = false;
   fvwb_xfer::Staging xfer;  // large copies from and to host arrays
   Tune tune{16, 2};
-  int short_rows = 0;       // strips of 1 or 2 rows instead (small grids; 0: tune.rows)
+  int short_rows = 0;       // strips of 1 or 2 rows stand for four (small grids; 0: tune.rows)
   std::string err;
 };
 
@@ -123,6 +123,22 @@ extern "C" int fvwb_params_reference_2d(fvwb_params* p, int32_t nx, int32_t ny, 
 static int alloc_dev(fvwb_ctx* h, void** ptr, size_t bytes) {
   FVWB_HIP(h, hipMalloc(ptr, bytes));
   return FVWB_OK;
+}
+
+// strips of the grid at `rows` rows and two columns per lane
+static long long strips(const fvwb_ctx* h, int rows) {
+  return (long long)((h->p.nx + 123) / 124) * ((h->p.ny + rows - 1) / rows);
+}
+// Four rows, the shortest shape a caller can ask for, are strips of one or two
+// (0: of four) on small grids; the same for a shape that was set as for the
+// default one, so that the shape get_launch returns is the one that runs.
+static int short_rows(const fvwb_ctx* h) {
+  if (h->tune.rows != 4 || h->tune.cpl != 2) return 0;
+  const int rows = short_strip_rows(strips(h, 1), strips(h, 2), false);
+  // FP64 strips of four that all run at once, two per SIMD, beat more than three
+  // of two rows: 69 against 73 us at 1000 x 800
+  if (h->p.precision == FVWB_FP64 && rows == 2 && strips(h, 2) > 3072 && strips(h, 4) <= 2048) return 0;
+  return rows;
 }
 
 extern "C" int fvwb_create(fvwb_handle* out, const fvwb_params* p) {
@@ -189,17 +205,15 @@ extern "C" int fvwb_create(fvwb_handle* out, const fvwb_params* p) {
   // steps took 54 and 63 us at 1200 x 900, 57 and 65 at 1500 x 900, but 70 and 68
   // at 1300^2, 96 and 92 at 1700^2.  The FP64 MUSCL kernels, two waves per SIMD,
   // were within 6 % either way and keep eight.
-  const long long cells = (long long)nx * ny, ntx = (nx + 123) / 124;
-  auto strips = [&](int rows) { return ntx * ((ny + rows - 1) / rows); };
-  auto length = [&](int rows) { return (strips(rows) + 1023) / 1024 * (2 * rows + 5); };
-  const bool fp64 = p->precision == FVWB_FP64, muscl = p->recon == FVWB_RECON_MUSCL_MINMOD;
-  h->tune.rows = cells >= (1ll << 24) ? 16 : cells >= (1ll << 22) ? 8 : cells < (1ll << 20) ? 4
-                 : !(fp64 && muscl) && length(4) < length(8) ? 4 : 8;
-  h->tune.cpl = 2;
-  h->short_rows = short_strip_rows(strips(1), strips(2), false);
-  // FP64 strips of four that all run at once, two per SIMD, beat more than three
-  // of two rows: 69 against 73 us at 1000 x 800
-  if (fp64 && h->short_rows == 2 && strips(2) > 3072 && strips(4) <= 2048) h->short_rows = 0;
+  h->tune = Tune{4, 2};
+  h->short_rows = short_rows(h);
+  if (!h->short_rows) {
+    const long long cells = (long long)nx * ny;
+    auto length = [&](int rows) { return (strips(h, rows) + 1023) / 1024 * (2 * rows + 5); };
+    const bool fp64 = p->precision == FVWB_FP64, muscl = p->recon == FVWB_RECON_MUSCL_MINMOD;
+    h->tune.rows = cells >= (1ll << 24) ? 16 : cells >= (1ll << 22) ? 8 : cells < (1ll << 20) ? 4
+                   : !(fp64 && muscl) && length(4) < length(8) ? 4 : 8;
+  }
   *out = h;
   return FVWB_OK;
 }
@@ -552,8 +566,8 @@ extern "C" int fvwb_set_launch(fvwb_handle h, int32_t rows_per_strip, int32_t co
   if (columns_per_lane != 2 && columns_per_lane != 4)
     return fail(h, FVWB_ERR_ARG, "columns_per_lane must be 2 or 4");
   h->tune.rows = rows_per_strip;
-  h->short_rows = 0;
   if (h->p.precision == FVWB_FP32) h->tune.cpl = columns_per_lane;
+  h->short_rows = short_rows(h);
   return FVWB_OK;
 }
 

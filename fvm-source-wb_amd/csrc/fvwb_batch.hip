@@ -73,8 +73,7 @@ struct fvwb_batch {
   int* d_tile_start = nullptr;
   int ntiles = 0;
   int rows = 8, cpl = 2, blocks = 0;    // launch shape (blocks 0 = automatic)
-  bool rows_set = false;                // by the caller: rows as given, else 4 may stand for 1 or 2
-  int strip_rows = 8;                   // rows of the strips as laid out
+  int strip_rows = 8;                   // rows of the strips as laid out (4 may stand for 1 or 2)
   int parity = 0;
   bool ready = false;
   fvwb_xfer::Staging xfer;  // large copies from and to host arrays
@@ -123,8 +122,11 @@ static int build_layout(fvwb_batch* h) {
   std::vector<int> start(h->ninst);
   long long total = 0;
   const int cpl = h->shared.precision == FVWB_FP64 ? 2 : h->cpl;
-  const bool free_rows = h->rows == 4 && cpl == 2 && !h->rows_set && h->shared.flux == FVWB_FLUX_HLL;
-  const int few = free_rows ? short_strip_rows(strips(h, 1), strips(h, 2), true) : 0;
+  // four rows stand for one or two on small batches, whoever asked for them
+  // (the default, a caller, the tuner or its cache), so that the shape that is
+  // reported is the one that runs; measured with HLL
+  const bool four = h->rows == 4 && cpl == 2 && h->shared.flux == FVWB_FLUX_HLL;
+  const int few = four ? short_strip_rows(strips(h, 1), strips(h, 2), true) : 0;
   h->strip_rows = few ? few : h->rows;
   for (int b = 0; b < h->ninst; ++b) {
     const fvwb_params& p = h->p[b];
@@ -486,7 +488,6 @@ extern "C" int fvwb_batch_set_launch(fvwb_batch_handle h, int32_t rows, int32_t 
   h->rows = rows;
   if (h->shared.precision == FVWB_FP32) h->cpl = cpl;
   h->blocks = blocks;
-  h->rows_set = true;
   return build_layout(h);
 }
 
@@ -568,7 +569,7 @@ extern "C" int fvwb_batch_autotune(fvwb_batch_handle h, int32_t trial_steps, con
     int rc = FVWB_OK;
     for (int ci = 0; ci < ncpl && rc == FVWB_OK; ++ci)
       for (int r : row_opts) {
-        h->rows = r; h->cpl = cpl_opts[ci]; h->blocks = 0; h->rows_set = false;
+        h->rows = r; h->cpl = cpl_opts[ci]; h->blocks = 0;
         rc = build_layout(h);
         if (rc) break;
         rc = enqueue_steps(h, 1, INFINITY);  // warm the kernel
@@ -598,7 +599,7 @@ extern "C" int fvwb_batch_autotune(fvwb_batch_handle h, int32_t trial_steps, con
     if (rc) return rc;
     cache_store(cache_path, key, rows, cpl, blocks, best / trial_steps);
   }
-  h->rows = rows; h->cpl = cpl; h->blocks = blocks; h->rows_set = false;
+  h->rows = rows; h->cpl = cpl; h->blocks = blocks;
   int rc = build_layout(h);
   if (rc) return rc;
   if (rows_out) *rows_out = rows;

@@ -156,8 +156,11 @@ int fvwb_get_stream(fvwb_handle h, void** stream);
 /* ---- launch shape (no counterpart in the reference) -------------------------
  * A wave owns a strip of 62*columns_per_lane columns and rows_per_strip rows.
  * columns_per_lane: 2 or 4 for FP32 (8- or 16-byte loads per lane and variable),
- * always 2 for FP64.  rows_per_strip: multiple of 4 in [4, 1024].  Results do not
- * depend on the shape; speed does. */
+ * always 2 for FP64.  rows_per_strip: multiple of 4 in [4, 1024]; 4 with two
+ * columns per lane asks for the shortest strips, which have one or two rows on
+ * grids small enough to leave the chip idle otherwise.  Setting the shape that
+ * fvwb_get_launch returns changes nothing.  Results do not depend on the shape;
+ * speed does. */
 int fvwb_set_launch(fvwb_handle h, int32_t rows_per_strip, int32_t columns_per_lane);
 int fvwb_get_launch(fvwb_handle h, int32_t* rows_per_strip, int32_t* columns_per_lane);
 
@@ -197,8 +200,10 @@ int fvwb_batch_get_time(fvwb_batch_handle h, int32_t inst, double* t, double* dt
 int fvwb_batch_get_stream(fvwb_batch_handle h, void** stream);
 /* Replay step pairs from a HIP graph (default on). */
 int fvwb_batch_use_graph(fvwb_batch_handle h, int32_t enable);
-/* Launch shape: rows per strip (multiple of 4), FP32 columns per lane (2/4),
- * persistent blocks (0 = one per four strips). */
+/* Launch shape: rows per strip (multiple of 4; 4 with two columns per lane and
+ * HLL: one or two rows on small batches), FP32 columns per lane (2/4),
+ * persistent blocks (0 = one per four strips).  ntiles of get_launch is the
+ * number of strips that run. */
 int fvwb_batch_set_launch(fvwb_batch_handle h, int32_t rows, int32_t cpl, int32_t blocks);
 int fvwb_batch_get_launch(fvwb_batch_handle h, int32_t* rows, int32_t* cpl, int32_t* blocks, int32_t* ntiles);
 /* Time `trial_steps` steps for each candidate shape on a saved copy of the

@@ -59,23 +59,46 @@ def test_batch_equals_single_instances_bitwise(prec, scheme):
 
 @pytest.mark.parametrize("prec", (fvwb.FP64, fvwb.FP32))
 def test_batch_of_short_strips_equals_single_instances_bitwise(prec):
-    """A batch whose strips have two rows, set to four and back by the tuner."""
+    """A batch whose strips have two rows against one on strips of eight and
+    each problem alone; the default shape, set again or taken by the tuner from
+    its cache, is the same strips."""
     sizes = [(300, 301), (248, 250), (40, 333), (310, 270)]
     say(f"case: batch of two-row strips prec={prec}")
     ps = inst_params(prec, sizes=sizes, gs=GS[:4])
     amps = np.array([1e-3, 1e-2, 5e-3, 1e-4])
-    with fvwb.Batch2D(ps) as bt, fvwb.Batch2D(ps) as b4:
-        b4.set_launch(4, 2)
-        for b in (bt, b4):
-            b.init_gaussian(amps)
-            b.advance(5)
-        assert bt.get_launch()[:2] == b4.get_launch()[:2] == (4, 2)
-        assert bt.get_launch()[3] > b4.get_launch()[3]
-        for k, p in enumerate(ps):
-            dev_s, (ts, dts, ns) = single_run(p, amps[k], 5)
-            for b in (bt, b4):
-                assert b.time(k) == (ts, dts, ns)
-                np.testing.assert_array_equal(b.download_deviation(k), dev_s)
+    two_rows = sum((nx + 123) // 124 * ((ny + 1) // 2) for nx, ny in sizes)
+    with fvwb.Batch2D(ps) as bt, fvwb.Batch2D(ps) as b8, tempfile.TemporaryDirectory() as td:
+        default = bt.get_launch()
+        assert default == (4, 2, 0, two_rows)
+        b8.set_launch(8, 2)
+        b8.init_gaussian(amps)
+        b8.advance(5)
+        cache = os.path.join(td, "tune.txt")
+        for how in ("default", "set", "tuned", "cached"):
+            bt.init_gaussian(amps)
+            if how == "set":
+                bt.set_launch(*default[:3])
+            elif how == "tuned":
+                rows, cpl = bt.autotune(1, cache)
+                # whatever it took, setting it gives the strips that were timed
+                took = bt.get_launch()
+                assert took[:2] == (rows, cpl)
+                bt.set_launch(*took[:3])
+                assert bt.get_launch() == took
+                with open(cache) as f:
+                    line = f.read()
+                with open(cache, "w") as f:
+                    f.write(line.replace(f"rows={rows} cpl={cpl}", "rows=4 cpl=2"))
+            elif how == "cached":
+                assert bt.autotune(1, cache) == (4, 2)
+            if how != "tuned":
+                assert bt.get_launch() == default, how
+            bt.advance(5)
+            for k, p in enumerate(ps):
+                dev_s, (ts, dts, ns) = single_run(p, amps[k], 5)
+                for b in (bt, b8):
+                    assert b.time(k) == (ts, dts, ns)
+                    np.testing.assert_array_equal(b.download_deviation(k), dev_s)
 
 
 def test_batch_fp64_matches_oracle():
