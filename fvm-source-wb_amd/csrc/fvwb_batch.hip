@@ -233,13 +233,17 @@ extern "C" int fvwb_batch_create(fvwb_batch_handle* out, int32_t ninst, const fv
     return bfail(nullptr, FVWB_ERR_HIP, "table upload failed");
   }
   // default launch shape: short strips (many waves), FP32 lanes own 2 columns.
-  // Four rows (or fewer, by build_layout) until they make four strips per SIMD:
-  // 2,500 of them ran 30 instances up to 400^2 in 61 us per FP32 step against
-  // 71 with eight rows, 4,350 of them 20 up to 700^2 in 91 against 89
+  // Four rows (or fewer, by build_layout) up to three strips per SIMD: 2,970 of
+  // them took 63 us per FP32 step against 72 with eight rows and 104 against 107 in
+  // FP64, 3,090 of them 81 against 72 and 124 against 106, 3,850 83 against 74 and
+  // 127 against 110.  One FP64 problem alone, whose strips all start together two
+  // per SIMD, takes four rows up to 2,560: 2,510 107 against 110, 2,880 113 against
+  // 107.
   // Rusanov batches keep eight: that flux rounds differently (by an ulp) upward
   // and downward, so its results depend on the strips, and an instance of a batch
   // equals the problem alone on strips of eight bit for bit
-  h->rows = s0.flux == FVWB_FLUX_HLL && strips(h, 4) <= 4096 ? 4 : 8;
+  const long long most = h->esize == 8 && h->ninst == 1 ? 2560 : 3072;
+  h->rows = s0.flux == FVWB_FLUX_HLL && strips(h, 4) <= most ? 4 : 8;
   h->cpl = 2;
   int rc = build_layout(h);
   if (rc) { g_batch_err = h->err; fvwb_batch_destroy(h); return rc; }

@@ -101,6 +101,19 @@ def test_batch_of_short_strips_equals_single_instances_bitwise(prec):
                     np.testing.assert_array_equal(b.download_deviation(k), dev_s)
 
 
+@pytest.mark.parametrize("prec,alone,most", ((fvwb.FP64, False, 3072), (fvwb.FP32, False, 3072), (fvwb.FP64, True, 2560),
+                                             (fvwb.FP32, True, 3072)))
+def test_default_rows_at_the_edge_of_what_runs_at_once(prec, alone, most):
+    """Strips of four rows up to the number that still pays, eight from the next
+    one on (four rows more are one more strip of four)."""
+    say(f"case: batch default rows prec={prec} alone={alone}")
+    for extra, rows in ((0, 4), (4, 8)):
+        sizes = [(100, 4 * most + extra)] if alone else [(100, most), (60, 2 * most), (124, most + extra)]
+        with fvwb.Batch2D(inst_params(prec, sizes=sizes, gs=GS[:len(sizes)])) as b:
+            tiles = sum((ny + rows - 1) // rows for _, ny in sizes)
+            assert b.get_launch() == (rows, 2, 0, tiles), extra
+
+
 def test_batch_fp64_matches_oracle():
     say("case: batch FP64 instances vs oracle")
     ps = inst_params(fvwb.FP64, sizes=SIZES[:4], gs=GS[:4])
