@@ -277,8 +277,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs<T>& a, const int tile
   // Even tile rows sweep upward, odd ones downward, so two vertically adjacent
   // tiles reach their shared halo rows at the same time and one of them finds
   // the rows in L2.  Both directions compute every face flux from the same two
-  // states in the same order (lower, upper), so the result does not depend on
-  // the direction (bit for bit with HLL; with Rusanov to an ulp).
+  // states in the same order (lower, upper), so the results of the two agree
+  // to an ulp (each is an instantiation whose products and sums may be fused
+  // differently: Rusanov's are from the first stage on, HLL's in FP32 now and
+  // then).
   // A ring of RING rows holds rows j, j+DIR, j+2DIR while row j is computed and
   // receives row j+(RING-1)DIR (one row in flight ahead of use); U^n uses a ring
   // of URING.  The body is unrolled RING times with rotated roles, so the rings

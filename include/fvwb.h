@@ -159,8 +159,10 @@ int fvwb_get_stream(fvwb_handle h, void** stream);
  * always 2 for FP64.  rows_per_strip: multiple of 4 in [4, 1024]; 4 with two
  * columns per lane asks for the shortest strips, which have one or two rows on
  * grids small enough to leave the chip idle otherwise.  Setting the shape that
- * fvwb_get_launch returns changes nothing.  Results do not depend on the shape;
- * speed does. */
+ * fvwb_get_launch returns changes nothing.  Results agree between shapes to
+ * rounding: a shape is another instantiation of the kernels, in which products
+ * and sums may be fused differently, by up to about one unit in the last place
+ * of the largest deviation per stage. */
 int fvwb_set_launch(fvwb_handle h, int32_t rows_per_strip, int32_t columns_per_lane);
 int fvwb_get_launch(fvwb_handle h, int32_t* rows_per_strip, int32_t* columns_per_lane);
 
@@ -179,7 +181,7 @@ int fvwb_copy_bandwidth(uint64_t bytes, int32_t reps, double* gbps);
  * One persistent launch per Runge-Kutta stage covers every strip of every
  * instance; step pairs are replayed from a HIP graph.  No counterpart in the
  * reference (it runs one problem per executable); each instance computes what
- * fvwb_create/fvwb_advance would compute for it alone. */
+ * fvwb_create/fvwb_advance would compute for it alone, to rounding (fvwb_set_launch). */
 typedef struct fvwb_batch* fvwb_batch_handle;
 int fvwb_batch_create(fvwb_batch_handle* h, int32_t ninst, const fvwb_params* per_inst);
 int fvwb_batch_destroy(fvwb_batch_handle h);

@@ -365,9 +365,10 @@ def test_advance_past_t_end_then_further(precision):
 @pytest.mark.parametrize("shape", [(4, 4), (125, 512), (125, 513), (130, 77), (700, 301), (1000, 1000)])
 def test_short_strips_equal_long_ones(shape, precision):
     """The one- and two-row strips that small grids get (1024 strips of one row
-    and one more, odd heights, the two-row range) against strips of eight: bit
-    for bit with HLL.  Rusanov rounds by an ulp of the deviation per stage
-    differently upward and downward, so there the bound is one per stage."""
+    and one more, odd heights, the two-row range) against strips of eight: the
+    same bits with HLL over these few steps.  Rusanov rounds by an ulp of the
+    deviation per stage differently upward and downward, so there the bound is
+    one per stage."""
     nx, ny = shape
     for flux in (fvwb.FLUX_HLL, fvwb.FLUX_RUSANOV):
         for recon, bc, integ, stages in ((fvwb.RECON_MUSCL_MINMOD, fvwb.BC_REFLECT, fvwb.SSPRK3, 3),
@@ -412,6 +413,27 @@ def test_shape_that_is_reported_is_the_one_that_runs(shape, precision):
             out.append((shape_now, s.download_deviation(), s.time()))
     assert out[0][0] == out[1][0] and out[0][2] == out[1][2]
     np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("precision", [fvwb.FP64, fvwb.FP32])
+@pytest.mark.parametrize("flux", [fvwb.FLUX_HLL, fvwb.FLUX_RUSANOV])
+def test_shapes_agree_to_rounding(flux, precision):
+    """Every launch shape over 40 steps: an ulp of the largest deviation per
+    stage, the bound that the header states."""
+    say(f"case: launch shapes agree flux={flux} precision={precision}")
+    p = fvwb.make_params(300, 301, flux=flux, recon=fvwb.RECON_MUSCL_MINMOD, bc=fvwb.BC_REFLECT,
+                         integrator=fvwb.SSPRK3, precision=precision, rho0=1.0, g=1.3)
+    out = []
+    for shape in (None, (4, 4), (8, 2), (12, 4), (64, 2), (1024, 4)):
+        with fvwb.Solver2D(p) as s:
+            if shape:
+                s.set_launch(*shape)
+            s.init_gaussian(1e-2, 0.4, 0.6, 80.0)
+            s.advance(40)
+            out.append(s.download_deviation())
+    eps = np.finfo(np.float64 if precision == fvwb.FP64 else np.float32).eps
+    for a in out[1:]:
+        np.testing.assert_allclose(a, out[0], rtol=0, atol=40 * 3 * eps * np.max(np.abs(out[0])))
 
 
 @pytest.mark.parametrize("nx,ny", [(511, 512), (512, 512), (512, 513), (1024, 1023), (1024, 1025), (1303, 1501)])
