@@ -127,10 +127,13 @@ constexpr int SLOTS = 64, SLOT_STRIDE = 16;     // 16 x 8 B = one 128-byte line
 // goes through LDS.  At 2049^2 the two updates with their element-wise passes,
 // copies and speed pass took 570 us per step as separate kernels with a thread
 // per cell; see the launch rule in strip_rows() for what they take now.
-template <int MODE>
+// PACKED: a grid of up to 30 columns leaves most lanes without a node, so the
+// wave holds several strips of rows side by side, in groups of 1 << lw >= nx + 2
+// lanes; the end lanes of a group own no cell and take nothing from the next.
+template <int MODE, bool PACKED>
 __global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const double* __restrict__ u0,
                                                        const double* __restrict__ u1, double* __restrict__ up,
-                                                       const double* __restrict__ diff, double dt, int rows,
+                                                       const double* __restrict__ diff, double dt, int rows, int lw,
                                                        const Clock* __restrict__ ck, double* __restrict__ o0,
                                                        double* __restrict__ o1,
                                                        unsigned long long* __restrict__ smax) {
@@ -144,18 +147,19 @@ __global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const
     u = odd ? u1 : u0;
     out = MODE == FIRST ? up : (odd ? o0 : o1);
   }
-  const int lane = threadIdx.x & 63;
-  const int strips = (g.nx + OWN - 1) / OWN;
-  const int tile = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b0 = tile / strips * rows;
-  if (b0 >= g.ny) return;
+  const int wave = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = PACKED ? threadIdx.x & ((1 << lw) - 1) : threadIdx.x & 63;
+  const int strips = PACKED ? 1 : (g.nx + OWN - 1) / OWN;
+  const int tile = PACKED ? (wave << (6 - lw)) + ((threadIdx.x & 63) >> lw) : wave;
+  if ((PACKED ? (wave << (6 - lw)) * rows : tile / strips * rows) >= g.ny) return;
+  const int b0 = tile / strips * rows;                   // of PACKED's last groups perhaps past the grid
   const int b1 = min(b0 + rows, g.ny);
   const int a = tile % strips * OWN - 1 + lane;          // this lane's node column
   const int ac = min(max(a, 0), g.nx - 1);
   const bool cell_x = a >= 0 && a < g.nx - 1;            // cell (a, .) exists
-  const bool own = lane >= 1 && lane <= OWN && a < g.nx;
+  const bool own = lane >= 1 && (PACKED || lane <= OWN) && a < g.nx;
   // a strip that touches no end of the grid has no copies to make
-  const bool inner = b0 > 1 && b1 < g.ny - 1 && tile % strips > 0 && tile % strips * OWN + OWN < g.nx - 1;
+  const bool inner = !PACKED && b0 > 1 && b1 < g.ny - 1 && tile % strips > 0 && tile % strips * OWN + OWN < g.nx - 1;
   const double dx = g.dx, dy = g.dy;
 
   auto load = [&](int r, Node& n) {
@@ -214,8 +218,10 @@ __global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const
 #pragma unroll
   for (int v = 0; v < 4; ++v) gsum[v] = P.g[v] + lane_from_right(P.g[v]);
 
-  // r: the row that closes cell row r-1 and completes node row r-1
-  for (int r = b0; r <= b1; ++r) {
+  // r: the row that closes cell row r-1 and completes node row r-1; every group
+  // of PACKED goes through as many rows
+  const int last = PACKED ? b0 + rows : b1;
+  for (int r = b0; r <= last; ++r) {
     Node N = next;
     load(r + 1, next);
     double nbase[4];
@@ -270,7 +276,7 @@ __global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const
       c3[v] = k3[v];
     }
     const int b = r - 1;
-    if (b >= b0 && own) {
+    if (b >= b0 && own && (!PACKED || b < b1)) {
       if (inner) {
         put(a, b, s, base);
       } else {
@@ -305,7 +311,7 @@ __global__ __launch_bounds__(256) void rd_sweep_kernel(Geo g, double area, const
   }
   if constexpr (MODE == SECOND) {
     for (int off = 32; off > 0; off >>= 1) speed_max = fmax(speed_max, __shfl_xor(speed_max, off));
-    if (lane == 0)
+    if ((threadIdx.x & 63) == 0)
       atomicMax(smax + (blockIdx.x % SLOTS) * SLOT_STRIDE, (unsigned long long)__double_as_longlong(speed_max));
   }
 }
@@ -445,27 +451,32 @@ extern "C" int fvwb_rd_create(fvwb_rd_handle* out, const fvwb_rd_params* p) {
   return FVWB_OK;
 }
 
-// Rows of a strip: about 4096 strips (two rounds of the two waves per SIMD that
+// Rows of a strip, of so many one-row strips: about 4096 strips (two rounds of the two waves per SIMD that
 // SECOND runs at), between 2 and 12 rows each.  A strip marches 2 rows more than
 // it owns, so short ones repeat work and long ones leave the chip idle on small
 // grids.  Measured us per step with 2 / 4 / 8 / 12 / 16 / 24 rows: 129^2 18.8 /
 // 24.6 / 37.3 / 49.9 / 62.7 / 87.3, 513^2 35.2 / 37.7 / 39.7 / 51.7 / 64.4 /
 // 89.1, 1025^2 80.4 / 73.1 / 77.2 / 75.7 / 93.5 / 90.1, 2049^2 275 / 231 / 209 /
 // 201 / 211 / 205.
-static int strip_rows(const Geo& g) {
-  const long long strips = (g.nx + OWN - 1) / OWN;
-  return (int)std::max(2LL, std::min(12LL, strips * g.ny / 4096));
-}
+static int strip_rows(long long strips) { return (int)std::max(2LL, std::min(12LL, strips / 4096)); }
 
 // One sweep: dudt of (u0, diff) into o0, or a pass of an 'RD1' step between the
-// state's two buffers.
+// state's two buffers.  Up to 30 columns the strips are packed into waves: 2 x
+// 200,000 nodes take 62 us per step (502 with a wave per strip, 400 with a thread
+// per cell), 16 x 100,000 172 (274 and 280), 30 x 1000 20 (21 and 36).
 template <int MODE>
 static int sweep(fvwb_rd* h, const double* u0, const double* u1, double* up, const double* diff, double dt,
                  const Clock* ck, double* o0, double* o1) {
-  const int rows = strip_rows(h->g);
-  const long long tiles = (long long)((h->p.nx + OWN - 1) / OWN) * ((h->p.ny + rows - 1) / rows);
-  hipLaunchKernelGGL(rd_sweep_kernel<MODE>, dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0, h->stream, h->g,
-                     h->g.dx * h->g.dy, u0, u1, up, diff, dt, rows, ck, o0, o1, h->d_smax);
+  const long long nx = h->p.nx, ny = h->p.ny;
+  int lw = 2;
+  while (lw < 6 && (1 << lw) < nx + 2) ++lw;
+  const bool packed = lw < 6;
+  const long long across = (nx + OWN - 1) / OWN, groups = 64 >> lw;
+  const int rows = strip_rows(packed ? ny / groups : across * ny);
+  const long long strips = across * ((ny + rows - 1) / rows), waves = packed ? (strips + groups - 1) / groups : strips;
+  hipLaunchKernelGGL((packed ? rd_sweep_kernel<MODE, true> : rd_sweep_kernel<MODE, false>),
+                     dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, h->stream, h->g, h->g.dx * h->g.dy, u0, u1, up,
+                     diff, dt, rows, lw, ck, o0, o1, h->d_smax);
   HIPR(h, hipGetLastError());
   return FVWB_OK;
 }

@@ -68,10 +68,14 @@ def test_run_matches_oracle(ninit, bc):
 
 
 @pytest.mark.parametrize("bc", [fvwb.RD_BC_TRANSMISSIVE, fvwb.RD_BC_PERIODIC])
-@pytest.mark.parametrize("shape", [(2, 2), (3, 2), (2, 3), (62, 3), (63, 4), (64, 5), (125, 2), (187, 25), (5, 300)])
+@pytest.mark.parametrize("shape", [(2, 2), (3, 2), (2, 3), (62, 3), (63, 4), (64, 5), (125, 2), (187, 25), (5, 300),
+                                   (2, 35), (3, 65), (6, 33), (7, 34), (14, 15), (15, 18), (30, 7), (31, 9), (2, 140000),
+                                   (30, 25000)])
 def test_strip_edges_and_buffer_parity(shape, bc, tmp_path):
     """Grids that end at, before and after a strip's 62 columns and its rows,
-    runs cut after an odd step, a drop-in call between them, and a checkpoint
+    narrow ones whose waves hold several strips (every group width, the last
+    group of a wave empty or in part past the grid, strips of two and of more
+    rows), runs cut after an odd step, a drop-in call between them, and a checkpoint
     of an odd step count loaded into a fresh handle."""
     nx, ny = shape
     say(f"case: rd strip edges {nx}x{ny} bc={bc}")
