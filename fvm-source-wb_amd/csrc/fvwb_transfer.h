@@ -14,7 +14,6 @@
 #include <algorithm>
 #include <cstddef>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 namespace fvwb_xfer {
@@ -108,7 +107,7 @@ inline hipError_t copy(Staging& s, void* dst, const void* src, size_t bytes, hip
   for (int t = 1; t < THREADS; ++t) {
     try {
       pool[t] = std::thread(work, t);
-    } catch (const std::system_error&) {           // no thread to be had: its share is done below
+    } catch (...) {                                // no thread or no memory for one: its share is done below
     }
   }
   work(0);
