@@ -63,8 +63,16 @@ inline bool known(const void* host) {
 
 template <bool DOWN>
 inline hipError_t copy(Staging& s, void* dst, const void* src, size_t bytes, hipStream_t st) {
-  int dev = 0;
-  if (bytes < (DOWN ? LEAST_DOWN : LEAST_UP) || known(DOWN ? dst : src) || hipGetDevice(&dev) != hipSuccess || !s.ready()) {
+  // the threads and the events belong to the stream's device, which need not be
+  // the caller's current one
+  int mine = 0, dev = 0;
+  bool staged = bytes >= (DOWN ? LEAST_DOWN : LEAST_UP) && !known(DOWN ? dst : src) &&
+                hipGetDevice(&mine) == hipSuccess && hipStreamGetDevice(st, &dev) == hipSuccess;
+  if (staged) {
+    staged = hipSetDevice(dev) == hipSuccess && s.ready();
+    if (!staged) (void)hipSetDevice(mine);
+  }
+  if (!staged) {
     (void)hipGetLastError();
     return hipMemcpyAsync(dst, src, bytes, DOWN ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, st);
   }
@@ -115,6 +123,7 @@ inline hipError_t copy(Staging& s, void* dst, const void* src, size_t bytes, hip
     if (pool[t].joinable()) pool[t].join();
     else work(t);
   }
+  (void)hipSetDevice(mine);
   for (hipError_t e : result)
     if (e != hipSuccess) return e;
   return hipSuccess;

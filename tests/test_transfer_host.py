@@ -101,7 +101,7 @@ void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 int main(int argc, char** argv) {
   const std::string what = argv[1];
-  Stream st{0, {}, 0, 0};
+  Stream st{what == "device" ? 1 : 0, {}, 0, 0};
   the_stream = &st;
   const size_t MB = 1 << 20;
   unsigned seed = 1;
@@ -124,6 +124,7 @@ int main(int argc, char** argv) {
         if (e != hipSuccess) return std::printf("down %zu: error %d\n", bytes, e), 1;
         hipStreamSynchronize(&st);
         if (up != down) return std::printf("%zu bytes differ\n", bytes), 1;
+        if (current != 0) return std::printf("the caller's device changed\n"), 1;
       }
     }
     if (what == "known") {
@@ -154,9 +155,10 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["plain", "known", "memory"])
+@pytest.mark.parametrize("what", ["plain", "known", "device", "memory"])
 def test_threaded_copies(program, what):
     """Copies of several sizes up and down through one set of slots: as they
-    are; of an array that the runtime knows; and with no memory for one of the helper threads."""
+    are; of an array that the runtime knows; with a stream of another device
+    than the current one; and with no memory for one of the helper threads."""
     r = subprocess.run([str(program), what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout, r.stderr)
