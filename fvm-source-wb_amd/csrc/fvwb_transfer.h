@@ -129,8 +129,9 @@ inline hipError_t copy(Staging& s, void* dst, const void* src, size_t bytes, hip
   return hipSuccess;
 }
 
-// Both are ordered on `st` like hipMemcpyAsync; the host array is read, or
-// filled, when they return.
+// Both are ordered on `st` like hipMemcpyAsync.  A pageable host array of these
+// sizes has been read, or filled, when they return; for any other the copy may
+// still be under way, so the caller waits for the stream in either case.
 inline hipError_t to_device(Staging& s, void* dst, const void* src, size_t bytes, hipStream_t st) {
   return copy<false>(s, dst, src, bytes, st);
 }
