@@ -104,7 +104,9 @@ int main(int argc, char** argv) {
   Stream st{what == "device" ? 1 : 0, {}, 0, 0};
   the_stream = &st;
   const size_t MB = 1 << 20;
+  pin_fails = what == "unpinned";
   unsigned seed = 1;
+  size_t most = 0;
   {
     fvwb_xfer::Staging s;
     for (size_t bytes : {size_t(3 * MB), size_t(9 * MB + 8), size_t(34 * MB - 24), size_t(150 * MB + 40), size_t(40 * MB)}) {
@@ -123,6 +125,9 @@ int main(int argc, char** argv) {
         new_countdown = -1;
         if (e != hipSuccess) return std::printf("down %zu: error %d\n", bytes, e), 1;
         hipStreamSynchronize(&st);
+        // what is pinned: about half the largest copy, at most 32 MB
+        most = std::max(most, bytes < 8 * MB ? 0 : std::min(bytes / 2 + MB, 32 * MB));
+        if (pinned > most) return std::printf("%zu bytes: %zu pinned\n", bytes, pinned), 1;
         if (up != down) return std::printf("%zu bytes differ\n", bytes), 1;
         if (current != 0) return std::printf("the caller's device changed\n"), 1;
       }
@@ -155,10 +160,11 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["plain", "known", "device", "memory"])
+@pytest.mark.parametrize("what", ["plain", "known", "device", "memory", "unpinned"])
 def test_threaded_copies(program, what):
-    """Copies of several sizes up and down through one set of slots: as they
-    are; of an array that the runtime knows; with a stream of another device
-    than the current one; and with no memory for one of the helper threads."""
+    """Copies of several sizes up and down through one set of slots, which are
+    no larger than the largest copy so far needs: as they are; of an array that the runtime knows; with a stream of another device
+    than the current one; with no memory for one of the helper threads; and with
+    none for the slots."""
     r = subprocess.run([str(program), what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout.strip() == "ok", (r.returncode, r.stdout, r.stderr)
