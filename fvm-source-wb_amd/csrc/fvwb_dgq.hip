@@ -31,9 +31,6 @@
 
 namespace dgq {
 
-#ifndef DGQ_WAVES
-#define DGQ_WAVES 3
-#endif
 constexpr int MAXO = 3;
 
 // Basis and quadrature of one set-up (order O = mx = my).
@@ -273,20 +270,6 @@ __device__ __forceinline__ void num_flux(const Geo& g, const double ul[4], const
       }
     }
   }
-}
-
-// get_boundary_conditions(index, 2) (:777-824) with one-based indices; the
-// reference passes dim = 2 for the x faces as well (:1338-1339), which is why
-// the residual needs nx == ny
-__device__ __forceinline__ int bc_index(int index, int n, int bc) {
-  if (bc == 1) {
-    if (index == 0) return n;
-    if (index == n + 1) return 1;
-  } else if (bc == 2 || bc == 3) {
-    if (index == 0) return 1;
-    if (index == n + 1) return n;
-  }
-  return index;
 }
 
 // grad_phi (:1599-1644) at one point
@@ -566,7 +549,7 @@ __global__ __launch_bounds__(256) void dgq_grad_kernel(int gcase, long long n, c
 // One stage on a tile of TX x TY cells, a wave per row of 16 cells:
 //   1. every lane expands its variable's modes to the cell's four traces
 //      (:1253-1314); waves 0 to 2 also do the one trace that each neighbour of
-//      the tile owes it (get_boundary_conditions at the domain's edge);
+//      the tile owes it (get_boundary_conditions :777-824 at the domain's edge);
 //   2. a thread per face point: the traces' fluxes (compute_flux_int :946-965)
 //      and compute_num_flux, written over the lower trace, which no other
 //      thread reads;
@@ -1279,6 +1262,8 @@ static void launch_speed(fvwb_dgq* h, const double* u, double* res, Clock* ck, d
 extern "C" int fvwb_dgq_create(fvwb_dgq_handle* out, const fvwb_dgq_params* p) {
   if (!out || !p) return failq(nullptr, FVWB_ERR_ARG, "NULL argument");
   *out = nullptr;
+  // the reference passes dim = 2 to get_boundary_conditions for the x faces as
+  // well (:1338-1339)
   if (p->nx < 1 || p->nx != p->ny)
     return failq(nullptr, FVWB_ERR_ARG,
                  "nx == ny >= 1 required (the reference's residual indexes the x faces with the y bounds)");

@@ -428,6 +428,7 @@ extern "C" int fvwb_rd_create(fvwb_rd_handle* out, const fvwb_rd_params* p) {
   *out = nullptr;
   if (p->nx < 2 || p->ny < 2) return failrd(nullptr, FVWB_ERR_ARG, "nx and ny must be >= 2");
   if ((long long)p->nx * p->ny > (1ll << 28)) return failrd(nullptr, FVWB_ERR_ARG, "more than 2^28 nodes");
+  // a limit of the interface, not of these launches: it has always been refused
   if (p->ny > 458745) return failrd(nullptr, FVWB_ERR_ARG, "ny must be <= 458745");
   if (p->bc != FVWB_RD_BC_PERIODIC && p->bc != FVWB_RD_BC_TRANSMISSIVE)
     return failrd(nullptr, FVWB_ERR_ARG, "bc must be 2 (periodic copies) or 3 (transmissive copies)");

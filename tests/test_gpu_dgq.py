@@ -119,11 +119,11 @@ def test_larger_grids_equal_oracle(order, kw):
         np.testing.assert_array_equal(s.download(), out)
 
 
-@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 34, 66])
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 32, 33, 34, 66])
 @pytest.mark.parametrize("order", [2, 3])
 def test_tile_edges_and_limited_states(n, order):
     """Grids that end inside, at and just past the stage kernel's 16 x 4 tiles
-    and either side of the one-launch speed reduction (64^2 cells), over every
+    and either side of the one-launch speed reduction (32^2 cells), over every
     solver, flux, boundary and source; the limiter on a state whose densities
     and pressures it has to scale, bit for bit."""
     k = 2 * n + order
